@@ -25,26 +25,12 @@ thread_local std::string g_tool_error;
 
 // ---- nearest centroid ----
 //
-// The distances ||x||^2 + ||c||^2 - 2 <x, c> come from a GEMM, in FP32 or from split-FP16
-// operands, each within (K + 32) 2^-24 ((||x|| + ||c||)^2) of the exact value (K products' and
-// sums' roundings, the norms' and the combination's). Where another centroid lies within the
-// two bounds of the smallest distance, the rows' candidates are evaluated again in FP64
-// (ties -> lower id), so the answer is the FP64 one whichever GEMM ran. On Gaussian mixtures
-// that is about one row in a hundred.
-
-// sum (x - c)^2 in FP64 over a wave's lanes (the same in every lane)
-__device__ __forceinline__ double wave_l2(const float *__restrict__ x, const float *__restrict__ c, uint32_t dim,
-                                          uint32_t lane) {
-    double s = 0.0;
-    for (uint32_t i = lane; i < dim; i += 64) {
-        const double d = (double)x[i] - (double)c[i];
-        s = fma(d, d, s);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        s += __shfl_xor(s, o, 64);
-    return s;
-}
+// The distances ||x||^2 + ||c||^2 - 2 <x, c> come from a GEMM on split-FP16 operands, each within
+// (K + 32) 2^-24 ((||x|| + ||c||)^2) of the exact value (K products' and sums' roundings, the
+// norms' and the combination's). Where another centroid lies within the two bounds of the
+// smallest distance, the row's candidates are evaluated again in FP64 (ties -> lower id), so
+// the answer is the FP64 one. On Gaussian mixtures that is about one row in a hundred. (The
+// FP32 GEMM's answer, where it runs instead, is its smallest distance.)
 
 // Two bounds above the smallest computed distance: no centroid beyond it can be the nearest.
 // A candidate's norm is at most ||x|| plus its distance.
@@ -55,14 +41,11 @@ __device__ __forceinline__ float nearest_cut(float best, float xnorm, uint32_t d
 
 // argmin over each row of dist [rows][k] (FP32 GEMM); ties -> lower index.
 __global__ __launch_bounds__(64) void row_argmin_kernel(const float *__restrict__ dist, uint32_t k,
-                                                        const float *__restrict__ x, const float *__restrict__ xn,
-                                                        const float *__restrict__ cent, uint32_t dim,
                                                         uint32_t *__restrict__ out) {
     const float *row = dist + (size_t)blockIdx.x * k;
-    const uint32_t lane = threadIdx.x;
     float best = FLT_MAX;
     uint32_t bi = 0xFFFFFFFFu;
-    for (uint32_t j = lane; j < k; j += 64) {
+    for (uint32_t j = threadIdx.x; j < k; j += 64) {
         const float v = row[j];
         if (v < best || (v == best && j < bi)) {
             best = v;
@@ -78,27 +61,7 @@ __global__ __launch_bounds__(64) void row_argmin_kernel(const float *__restrict_
             bi = oi;
         }
     }
-    if (bi != 0xFFFFFFFFu) {
-        const float *xr = x + (size_t)blockIdx.x * dim;
-        const float cut = nearest_cut(best, xn[blockIdx.x], dim);
-        double exact = -1.0;  // of bi, once it is needed
-        for (uint32_t j0 = 0; j0 < k; j0 += 64) {
-            const uint32_t j = j0 + lane;
-            unsigned long long m = __ballot(j < k && j != bi && row[j < k ? j : 0] <= cut);
-            while (m) {
-                const uint32_t c = j0 + (uint32_t)__builtin_ctzll(m);
-                m &= m - 1;
-                if (exact < 0.0)
-                    exact = wave_l2(xr, cent + (size_t)bi * dim, dim, lane);
-                const double d = wave_l2(xr, cent + (size_t)c * dim, dim, lane);
-                if (d < exact || (d == exact && c < bi)) {
-                    exact = d;
-                    bi = c;
-                }
-            }
-        }
-    }
-    if (lane == 0)
+    if (threadIdx.x == 0)
         out[blockIdx.x] = bi == 0xFFFFFFFFu ? 0u : bi;
 }
 
@@ -142,8 +105,50 @@ __global__ __launch_bounds__(256) void nearest_rows_kernel(const unsigned long l
         list[atomicAdd(count, 1u)] = row;
 }
 
+// sum (x - c)^2 in FP64 for N centroids at a time by a group of eight lanes (the same in all of
+// them). Aligned rows of whole quads are read four values at a time.
+template <int N>
+__device__ __forceinline__ void group_l2(const float *__restrict__ x, const float *const (&c)[N], uint32_t dim,
+                                         uint32_t gl, double (&s)[N]) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        s[j] = 0.0;
+    const auto term = [](float a, float b, double acc) {
+        const double d = (double)a - (double)b;
+        return fma(d, d, acc);
+    };
+    if (dim % 4 == 0) {
+        for (uint32_t i = 4 * gl; i < dim; i += 32) {
+            const float4 a = *reinterpret_cast<const float4 *>(x + i);
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const float4 b = *reinterpret_cast<const float4 *>(c[j] + i);
+                s[j] = term(a.x, b.x, s[j]);
+                s[j] = term(a.y, b.y, s[j]);
+                s[j] = term(a.z, b.z, s[j]);
+                s[j] = term(a.w, b.w, s[j]);
+            }
+        }
+    } else {
+        for (uint32_t i = gl; i < dim; i += 8) {
+            const float a = x[i];
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+                s[j] = term(a, c[j][i], s[j]);
+        }
+    }
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            s[j] += __shfl_xor(s[j], o, 64);
+}
+
 // The listed rows' nearest centroid in FP64 over the candidates: a tile's best, or all 128
-// centroids of a tile whose second smallest distance is a candidate too. A workgroup per row.
+// centroids of a tile whose second smallest distance is a candidate too. A workgroup per row,
+// its 32 groups of eight lanes a centroid each (four where a whole tile is evaluated). What
+// bounds it, when few rows are listed, is the chain of a row: 12 MB of 256-dimensional rows,
+// k = 256: one wave a centroid, 32 of them in turn, 159 us; this shape 8.6 us.
 __global__ __launch_bounds__(256) void nearest_exact_kernel(const unsigned long long *__restrict__ best,
                                                             const uint32_t *__restrict__ second, uint32_t tiles,
                                                             const float *__restrict__ x, const float *__restrict__ xn,
@@ -151,49 +156,84 @@ __global__ __launch_bounds__(256) void nearest_exact_kernel(const unsigned long 
                                                             const uint32_t *__restrict__ list,
                                                             const uint32_t *__restrict__ count,
                                                             uint32_t *__restrict__ out) {
+    __shared__ unsigned long long s_min[4];
     __shared__ double s_d[4];
     __shared__ uint32_t s_c[4];
-    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x & 63, n = *count;
+    __shared__ uint32_t s_item[256], s_whole[256], s_items, s_wholes;
+    const uint32_t t = threadIdx.x, wave = t / 64, lane = t & 63, group = t / 8, gl = t & 7, n = *count;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const uint32_t row = list[i];
         const unsigned long long *b = best + (size_t)row * tiles;
         const uint32_t *sec = second + (size_t)row * tiles;
         unsigned long long mine = ~0ull;
-        for (uint32_t t = lane; t < tiles; t += 64)
-            mine = min(mine, b[t]);
+        for (uint32_t j = t; j < tiles; j += 256)
+            mine = min(mine, b[j]);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1)
             mine = min(mine, (unsigned long long)__shfl_xor(mine, o, 64));
+        if (lane == 0)
+            s_min[wave] = mine;
+        __syncthreads();
+        mine = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
         const float cut = nearest_cut(float_of_key((uint32_t)(mine >> 32)), xn[row], dim);
         const float *xr = x + (size_t)row * dim;
         double bd = __longlong_as_double(0x7FF0000000000000ll);
         uint32_t bc = 0xFFFFFFFFu;
-        const auto try_one = [&](uint32_t c) {
-            const double d = wave_l2(xr, cent + (size_t)c * dim, dim, lane);
+        const auto take = [&](double d, uint32_t c) {
             if (d < bd || (d == bd && c < bc)) {
                 bd = d;
                 bc = c;
             }
         };
-        for (uint32_t t = wave; t < tiles; t += 4) {
-            if (float_of_key(sec[t]) <= cut) {
-                for (uint32_t c = 128 * t; c < min(k, 128 * t + 128); ++c)
-                    try_one(c);
-            } else if (float_of_key((uint32_t)(b[t] >> 32)) <= cut) {
-                try_one((uint32_t)b[t]);
+        // 256 tiles at a time: single candidates and whole tiles to two lists
+        for (uint32_t t0 = 0; t0 < tiles; t0 += 256) {
+            if (t == 0)
+                s_items = s_wholes = 0;
+            __syncthreads();
+            const uint32_t tile = t0 + t;
+            if (tile < tiles) {
+                if (float_of_key(sec[tile]) <= cut)
+                    s_whole[atomicAdd(&s_wholes, 1u)] = tile;
+                else if (float_of_key((uint32_t)(b[tile] >> 32)) <= cut)
+                    s_item[atomicAdd(&s_items, 1u)] = (uint32_t)b[tile];
             }
+            __syncthreads();
+            const uint32_t items = s_items, wholes = s_wholes;
+            for (uint32_t j = group; j < items; j += 32) {
+                const float *const c[1] = {cent + (size_t)s_item[j] * dim};
+                double d[1];
+                group_l2<1>(xr, c, dim, gl, d);
+                take(d[0], s_item[j]);
+            }
+            for (uint32_t j = 0; j < wholes; ++j) {
+                const uint32_t c0 = 128 * s_whole[j] + group;
+                const float *c[4];
+                double d[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    c[u] = cent + (size_t)min(c0 + 32 * u, k - 1) * dim;
+                group_l2<4>(xr, c, dim, gl, d);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (c0 + 32 * u < k)
+                        take(d[u], c0 + 32 * u);
+            }
+            __syncthreads();  // the lists are written again
+        }
+#pragma unroll
+        for (int o = 32; o >= 8; o >>= 1) {
+            const double od = __shfl_xor(bd, o, 64);
+            const uint32_t oc = __shfl_xor(bc, o, 64);
+            take(od, oc);
         }
         if (lane == 0) {
             s_d[wave] = bd;
             s_c[wave] = bc;
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
+        if (t == 0) {
             for (int w = 1; w < 4; ++w)
-                if (s_d[w] < bd || (s_d[w] == bd && s_c[w] < bc)) {
-                    bd = s_d[w];
-                    bc = s_c[w];
-                }
+                take(s_d[w], s_c[w]);
             if (bc != 0xFFFFFFFFu)
                 out[row] = bc;
         }
@@ -273,7 +313,7 @@ int assign_rows(const float *d_x, size_t n, uint32_t dim, const float *d_c, cons
         const uint32_t rows = (uint32_t)std::min(chunk, n - b);
         launch_row_norms(d_x + b * dim, rows, dim, d_xn, s);
         launch_dist_gemm(d_x + b * dim, d_xn, d_c, d_cn, rows, k, dim, d_dist, s);
-        row_argmin_kernel<<<rows, 64, 0, s>>>(d_dist, k, d_x + b * dim, d_xn, d_c, dim, d_assign + b);
+        row_argmin_kernel<<<rows, 64, 0, s>>>(d_dist, k, d_assign + b);
     }
     TCHK(hipGetLastError());
     return CORA_OK;

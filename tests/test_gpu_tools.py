@@ -7,6 +7,7 @@ distances of the returned neighbours against the FP64 optimum, to FP32 accuracy.
 """
 import ctypes
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -264,3 +265,27 @@ def test_assign_is_the_fp64_nearest(n, dim, k):
     assert np.all(got <= best * (1 + dim * 2.0 ** -50))
     first = (d <= best[:, None]).argmax(1)
     assert np.array_equal(a[got == best], first[got == best])
+
+
+def call_seconds(f, n=15):
+    f()
+    best = float("inf")
+    for _ in range(n):
+        t = time.perf_counter()
+        f()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+def test_settling_one_row_costs_little():
+    """A row half-way between two centroids is evaluated again in FP64, over the 128 centroids of
+    their tile: a call that holds one takes about as long as one that holds none."""
+    rng = np.random.default_rng(77)
+    n, dim, k = 1024, 1024, 128
+    c = rng.standard_normal((k, dim)).astype(np.float32)
+    x = (c[rng.integers(0, k, n)] + 0.1 * rng.standard_normal((n, dim))).astype(np.float32)
+    y = x.copy()
+    y[5] = (c[0] + c[1]) / 2
+    none, one = (call_seconds(lambda v=v: ca.gpu_assign(v, c)) for v in (x, y))
+    say(f"[tools] assign {n} x {dim}, k {k}: no row settled {none * 1e3:.3f} ms, one {one * 1e3:.3f} ms")
+    assert one <= 1.3 * none
