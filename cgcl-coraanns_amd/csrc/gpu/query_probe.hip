@@ -12,6 +12,7 @@
 #include <math.h>
 
 #include "engine_internal.h"
+#include "tile_order.h"
 
 namespace cora {
 namespace {
@@ -372,9 +373,8 @@ constexpr int kEs = kHT + 4;  // LDS row stride (floats) of the epilogue's half 
 // the MFMAs; 32 KB of LDS and 158 VGPRs let three workgroups share a CU, which hides the
 // load latency better than two double-buffered ones). MFMA 16x16x32 operand layout: lane l
 // supplies A[l % 16][8 (l / 16) .. + 7] and B[8 (l / 16) .. + 7][l % 16], and holds
-// D[4 (l / 16) + r][l % 16]. Tile order: XCD x (blockIdx.x % 8) owns column tiles
-// [x ncx, (x + 1) ncx), swept by groups of four row tiles, so the workgroups resident on
-// an XCD share their operand tiles in its L2.
+// D[4 (l / 16) + r][l % 16]. Tile order: tile_order.h (modes 2 and 3 by columns; ncx: the
+// column tiles an XCD owns, 0: by rows).
 template <int kMode, int kSlots = kProbeSlots>
 __global__ __launch_bounds__(256, 3) void dist_gemm_f16x3_kernel(
     const _Float16 *__restrict__ Ah, const _Float16 *__restrict__ Al, const float *__restrict__ as,
@@ -387,9 +387,9 @@ __global__ __launch_bounds__(256, 3) void dist_gemm_f16x3_kernel(
     constexpr size_t kLdsBytes = kMode == 2 && kHalfBytes > kOperandBytes ? kHalfBytes : kOperandBytes;
     __shared__ __align__(16) unsigned char s_raw[kLdsBytes];
     half8_t(*S)[kHT * 4] = reinterpret_cast<half8_t(*)[kHT * 4]>(s_raw);  // [Ah, Al, Bh, Bl][row x group]
-    const uint32_t xcd = blockIdx.x % kNumXcd, bi = blockIdx.x / kNumXcd;
-    const uint32_t grp = bi / (4 * ncx), within = bi % (4 * ncx);
-    const uint32_t n0 = (xcd * ncx + within / 4) * kHT;
+    uint32_t rt, ct;
+    tile_of(blockIdx.x, ncx, (N + kHT - 1) / kHT, rt, ct);
+    const uint32_t n0 = ct * kHT;
     const uint32_t Me = kMode == 3 ? min(M, *mcount) : M;
     if (n0 >= N)
         return;  // the whole workgroup: padding of the tile grid
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(256, 3) void dist_gemm_f16x3_kernel(
             }
         }
     };
-    const uint32_t m_first = (grp * 4 + within % 4) * kHT;
+    const uint32_t m_first = rt * kHT;
     if constexpr (kMode != 3) {
         if (m_first < M)
             row_tile(m_first);
@@ -1888,12 +1888,11 @@ void launch_dist_gemm_f16x3_rows(const uint16_t *qhi, const uint16_t *qlo, const
                                  uint32_t nq, uint32_t nl, uint32_t P, float *dist, hipStream_t s) {
     if (!nq || !nl)
         return;
-    const uint32_t nrt = (nq + kHT - 1) / kHT, nct = (nl + kHT - 1) / kHT;
-    const uint32_t ncx = (nct + kNumXcd - 1) / kNumXcd, groups = (nrt + 3) / 4;
-    dist_gemm_f16x3_kernel<1><<<kNumXcd * ncx * 4 * groups, 256, 0, s>>>(
+    const TileOrder o = tile_order((nq + kHT - 1) / kHT, (nl + kHT - 1) / kHT);
+    dist_gemm_f16x3_kernel<1><<<o.blocks, 256, 0, s>>>(
         reinterpret_cast<const _Float16 *>(qhi), reinterpret_cast<const _Float16 *>(qlo), qscale,
         reinterpret_cast<const _Float16 *>(chi), reinterpret_cast<const _Float16 *>(clo), cscale, dist, nq, nl, P,
-        qnorm, cnorm, ncx, groups * 4 * kHT, nullptr, nullptr, nullptr, 0);
+        qnorm, cnorm, o.cols, 0, nullptr, nullptr, nullptr, 0);
 }
 
 uint32_t nearest_tiles(uint32_t nl) { return (nl + kHT - 1) / kHT; }
@@ -1904,13 +1903,12 @@ void launch_nearest_gemm(const uint16_t *xhi, const uint16_t *xlo, const float *
                          hipStream_t s) {
     if (!rows || !nl)
         return;
-    const uint32_t nrt = (rows + kHT - 1) / kHT, nct = nearest_tiles(nl);
-    const uint32_t ncx = (nct + kNumXcd - 1) / kNumXcd, groups = (nrt + 3) / 4;
-    dist_gemm_f16x3_kernel<4><<<kNumXcd * ncx * 4 * groups, 256, 0, s>>>(
+    const uint32_t nct = nearest_tiles(nl);
+    const TileOrder o = tile_order((rows + kHT - 1) / kHT, nct);
+    dist_gemm_f16x3_kernel<4><<<o.blocks, 256, 0, s>>>(
         reinterpret_cast<const _Float16 *>(xhi), reinterpret_cast<const _Float16 *>(xlo), xscale,
         reinterpret_cast<const _Float16 *>(chi), reinterpret_cast<const _Float16 *>(clo), cscale,
-        reinterpret_cast<float *>(second), rows, nl, K, xnorm, cnorm, ncx, groups * 4 * kHT, nullptr, nullptr, best,
-        nct);
+        reinterpret_cast<float *>(second), rows, nl, K, xnorm, cnorm, o.cols, 0, nullptr, nullptr, best, nct);
 }
 
 bool fused_probe_supported(uint32_t nl, uint32_t nprobe) {
@@ -2012,13 +2010,12 @@ void launch_rotate_f16x3_rows(const uint16_t *xhi, const uint16_t *xlo, const fl
                               hipStream_t s) {
     if (!rows)
         return;
-    const uint32_t nrt = (rows + kHT - 1) / kHT, nct = (P + kHT - 1) / kHT;
-    const uint32_t ncx = (nct + kNumXcd - 1) / kNumXcd, groups = (nrt + 3) / 4;
+    const TileOrder o = tile_order((rows + kHT - 1) / kHT, (P + kHT - 1) / kHT);
     const _Float16 *xh = reinterpret_cast<const _Float16 *>(xhi);
     const _Float16 *rh = reinterpret_cast<const _Float16 *>(rthl);
-    dist_gemm_f16x3_kernel<0><<<kNumXcd * ncx * 4 * groups, 256, 0, s>>>(
+    dist_gemm_f16x3_kernel<0><<<o.blocks, 256, 0, s>>>(
         xh, reinterpret_cast<const _Float16 *>(xlo), xscale, rh, rh + (size_t)P * dim, rtscale, out, rows, P, dim,
-        nullptr, nullptr, ncx, groups * 4 * kHT, nullptr, nullptr, nullptr, 0);
+        nullptr, nullptr, o.cols, 0, nullptr, nullptr, nullptr, 0);
 }
 
 // ---- big-k select (nprobe > kSelectMaxProbe, up to 65,536): one 1024-thread block per
