@@ -1,16 +1,18 @@
 // Large host arrays to the device and back for the index-build tools, whose callers hold
 // ordinary (pageable) arrays.
 //
-// The runtime copies a pageable array through its own staging at ~30 GB/s while the caller
-// waits; a DMA from page-locked memory runs at 57 GB/s. Here a few host threads copy 4 MiB pieces
-// into page-locked buffers (one thread copies 10-15 GB/s) and queue their DMAs on a stream of
-// their own, and the caller's kernels for a chunk of rows are launched as soon as the chunk is
-// queued, so that they run while the following chunks travel. Measured with the kernels of
-// this repository: assign 300,000 x 768, k = 8,192 (922 MB up) 50 -> 24.8 ms a call.
+// The runtime copies a pageable array to the device at 36 GB/s (28 from 64 MiB) and back at
+// 17 GB/s while the caller waits; a DMA from page-locked memory runs at 57 GB/s. Here a few
+// host threads copy 4 MiB pieces into page-locked buffers (one thread copies 10-15 GB/s) and
+// queue their DMAs on a stream of their own, and the caller's kernels for a chunk of rows are
+// launched as soon as the chunk is queued, so that they run while the following chunks travel.
 //
-// A staging set (48 MiB of page-locked memory, two streams, events) is taken for one call and
-// given back after it; at most kKeepSets are kept for later calls, so calls from several threads
-// never share one.
+// A staging set (threads, their page-locked buffers, a stream, events) belongs to one call
+// from its first large copy to its end; at most kKeepSets a device are kept for later calls, so
+// calls from several host threads never share one. The threads of a set sleep between copies,
+// and sleep while they wait for a buffer's DMA (hipEventBlockingSync): with threads started by
+// each copy, and waits that spun, repeated calls took one or two scheduler ticks of 4 ms longer
+// now and then (assign 12 MB 0.75 or 4.0 ms; the copy alone shows none of it).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -20,6 +22,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <mutex>
+#include <new>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -27,50 +30,131 @@
 namespace cora {
 
 constexpr size_t kPieceBytes = size_t{4} << 20;
-constexpr int kCopyThreads = 6;
-constexpr size_t kKeepSets = 2;
-// below this the runtime's copy is as fast as starting the threads
-constexpr size_t kStagedMinBytes = size_t{8} << 20;
+constexpr int kCopyThreads = 4;  // 3, 4 and 6 copy alike
+constexpr int kKeepSets = 2;
+// Below these the runtime's copy is as fast. Up: plain 0.24 / 0.46 / 0.94 / 2.58 ms for 8, 16, 32
+// and 64 MiB, staged 0.27 / 0.46 / 0.82 / 1.58. Down: plain 0.25 / 0.49 / 0.98 / 2.03 for 4, 8, 16
+// and 32 MiB, staged 0.30 / 0.38 / 0.58 / 0.99.
+constexpr size_t kStagedUpBytes = size_t{32} << 20;
+constexpr size_t kStagedDownBytes = size_t{8} << 20;
 
 struct StagingSet {
     int device = 0;
-    hipStream_t up = nullptr, down = nullptr;
-    hipEvent_t fence = nullptr;
+    StagingSet *next = nullptr;  // in the pool
+    hipStream_t stream = nullptr;
+    hipEvent_t mark = nullptr;
     void *buf[2 * kCopyThreads] = {};
     hipEvent_t ev[2 * kCopyThreads] = {};
 
     bool create(int dev) {
         device = dev;
-        if (hipStreamCreateWithFlags(&up, hipStreamNonBlocking) != hipSuccess ||
-            hipStreamCreateWithFlags(&down, hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&fence, hipEventDisableTiming) != hipSuccess)
+        if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess ||
+            hipEventCreateWithFlags(&mark, hipEventDisableTiming) != hipSuccess)
             return false;
         for (int i = 0; i < 2 * kCopyThreads; ++i)
             if (hipHostMalloc(&buf[i], kPieceBytes, hipHostMallocDefault) != hipSuccess ||
-                hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess)
+                hipEventCreateWithFlags(&ev[i], hipEventDisableTiming | hipEventBlockingSync) != hipSuccess)
                 return false;
-        return true;
+        for (; threads_ < kCopyThreads; ++threads_) {
+            try {
+                thread_[threads_] = std::thread([this, t = threads_] { serve(t); });
+            } catch (const std::system_error &) {
+                break;
+            }
+        }
+        return threads_ > 0;
     }
-    void destroy() {
+    ~StagingSet() {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            quit_ = true;
+        }
+        wake_.notify_all();
+        for (int t = 0; t < threads_; ++t)
+            thread_[t].join();
         for (int i = 0; i < 2 * kCopyThreads; ++i) {
             if (ev[i])
                 (void)hipEventDestroy(ev[i]);
             if (buf[i])
                 (void)hipHostFree(buf[i]);
         }
-        if (fence)
-            (void)hipEventDestroy(fence);
-        if (up)
-            (void)hipStreamDestroy(up);
-        if (down)
-            (void)hipStreamDestroy(down);
+        if (mark)
+            (void)hipEventDestroy(mark);
+        if (stream)
+            (void)hipStreamDestroy(stream);
     }
+
+    // work(t) on the threads t = 0 .. min(pieces, threads) - 1; join() ends the job. work lives
+    // until then and throws nothing.
+    template <class W>
+    void start(W &work, size_t pieces) {
+        std::lock_guard<std::mutex> lock(mu_);
+        arg_ = &work;
+        fn_ = [](void *w, int t) { (*static_cast<W *>(w))(t); };
+        want_ = active_ = (int)std::min<size_t>(threads_, pieces);
+        ++job_;
+        wake_.notify_all();
+    }
+    void join() {
+        std::unique_lock<std::mutex> lock(mu_);
+        done_.wait(lock, [&] { return active_ == 0; });
+    }
+
+  private:
+    void serve(int t) {
+        uint64_t seen = 0;
+        std::unique_lock<std::mutex> lock(mu_);
+        for (;;) {
+            wake_.wait(lock, [&] { return quit_ || job_ != seen; });
+            if (quit_)
+                return;
+            seen = job_;
+            if (t >= want_)
+                continue;
+            lock.unlock();
+            fn_(arg_, t);
+            lock.lock();
+            if (--active_ == 0)
+                done_.notify_all();
+        }
+    }
+
+    std::mutex mu_;
+    std::condition_variable wake_, done_;
+    uint64_t job_ = 0;
+    int want_ = 0, active_ = 0, threads_ = 0;
+    bool quit_ = false;
+    void *arg_ = nullptr;
+    void (*fn_)(void *, int) = nullptr;
+    std::thread thread_[kCopyThreads];
 };
 
-// The idle sets. Never destroyed: at the process's end the runtime may already be gone.
+// The idle sets. Never destroyed: at the process's end the runtime may already be gone (the
+// sets' threads sleep until then).
 struct StagingPool {
     std::mutex mu;
-    std::vector<StagingSet *> idle;
+    StagingSet *idle = nullptr;
+    StagingSet *take(int device) {
+        std::lock_guard<std::mutex> lock(mu);
+        for (StagingSet **p = &idle; *p; p = &(*p)->next)
+            if ((*p)->device == device) {
+                StagingSet *s = *p;
+                *p = s->next;
+                return s;
+            }
+        return nullptr;
+    }
+    bool keep(StagingSet *s) {
+        std::lock_guard<std::mutex> lock(mu);
+        int n = 0;
+        for (StagingSet *i = idle; i; i = i->next)
+            n += i->device == s->device;
+        if (n >= kKeepSets)
+            return false;
+        s->next = idle;
+        idle = s;
+        return true;
+    }
 };
 inline StagingPool &staging_pool() {
     static StagingPool *pool = new StagingPool();
@@ -86,18 +170,9 @@ class Staging {
         if (!set_)
             return;
         // nothing of this call may still use the buffers
-        (void)hipStreamSynchronize(set_->up);
-        (void)hipStreamSynchronize(set_->down);
-        StagingPool &pool = staging_pool();
-        {
-            std::lock_guard<std::mutex> lock(pool.mu);
-            if (pool.idle.size() < kKeepSets) {
-                pool.idle.push_back(set_);
-                return;
-            }
-        }
-        set_->destroy();
-        delete set_;
+        (void)hipStreamSynchronize(set_->stream);
+        if (!staging_pool().keep(set_))
+            delete set_;
     }
     Staging(const Staging &) = delete;
     Staging &operator=(const Staging &) = delete;
@@ -110,11 +185,16 @@ class Staging {
     hipError_t upload(const void *src, void *dst, size_t bytes, size_t chunk_bytes, int &rc, F launch) {
         rc = 0;
         const size_t nchunks = (bytes + chunk_bytes - 1) / chunk_bytes;
-        if (bytes >= kStagedMinBytes && acquire()) {
-            bool ran = false;
-            const hipError_t r = staged_upload(src, dst, bytes, chunk_bytes, nchunks, rc, launch, ran);
-            if (ran)
-                return r;
+        if (bytes >= kStagedUpBytes && acquire()) {
+            std::vector<uint32_t> left;  // pieces of each chunk that are not queued yet
+            bool room = true;
+            try {
+                left.resize(nchunks);
+            } catch (const std::bad_alloc &) {
+                room = false;
+            }
+            if (room)
+                return staged_upload(src, dst, bytes, chunk_bytes, left, rc, launch);
         }
         for (size_t c = 0; c < nchunks; ++c) {
             const size_t o = c * chunk_bytes, len = std::min(chunk_bytes, bytes - o);
@@ -127,19 +207,11 @@ class Staging {
         }
         return hipSuccess;
     }
-    hipError_t upload(const void *src, void *dst, size_t bytes) {
-        int rc;
-        return upload(src, dst, bytes, std::max<size_t>(1, bytes), rc, [](size_t, size_t) { return 0; });
-    }
 
     // src (device, written by work already on the null stream) to dst [bytes]; complete on return.
     hipError_t download(const void *src, void *dst, size_t bytes) {
-        if (bytes >= kStagedMinBytes && acquire()) {
-            bool ran = false;
-            const hipError_t r = staged_download(src, dst, bytes, ran);
-            if (ran)
-                return r;
-        }
+        if (bytes >= kStagedDownBytes && acquire())
+            return staged_download(src, dst, bytes);
         return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
     }
 
@@ -148,87 +220,53 @@ class Staging {
         if (set_ || tried_)
             return set_ != nullptr;
         tried_ = true;
-        StagingPool &pool = staging_pool();
-        {
-            std::lock_guard<std::mutex> lock(pool.mu);
-            for (size_t i = 0; i < pool.idle.size(); ++i)
-                if (pool.idle[i]->device == device_) {
-                    set_ = pool.idle[i];
-                    pool.idle.erase(pool.idle.begin() + (long)i);
-                    return true;
-                }
-        }
-        set_ = new StagingSet();
-        if (!set_->create(device_)) {
+        set_ = staging_pool().take(device_);
+        if (set_)
+            return true;
+        set_ = new (std::nothrow) StagingSet();
+        if (set_ && !set_->create(device_)) {
             (void)hipGetLastError();
-            set_->destroy();
             delete set_;
             set_ = nullptr;
         }
         return set_ != nullptr;
     }
 
-    // up to kCopyThreads threads running work(index); the number that could be started
-    template <class W>
-    static int start(std::vector<std::thread> &threads, size_t pieces, W work) {
-        const int want = (int)std::min<size_t>(kCopyThreads, pieces);
-        for (int t = 0; t < want; ++t) {
-            try {
-                threads.emplace_back(work, t);
-            } catch (const std::system_error &) {
-                break;
-            }
-        }
-        return (int)threads.size();
-    }
-
     template <class F>
-    hipError_t staged_upload(const void *src, void *dst, size_t bytes, size_t chunk_bytes, size_t nchunks, int &rc,
-                             F &launch, bool &ran) {
-        struct Piece {
-            size_t off, len, chunk;
-        };
-        std::vector<Piece> pieces;
-        std::vector<uint32_t> left(nchunks, 0);
+    hipError_t staged_upload(const void *src, void *dst, size_t bytes, size_t chunk_bytes, std::vector<uint32_t> &left,
+                             int &rc, F &launch) {
+        const size_t nchunks = left.size();
+        const size_t per = (chunk_bytes + kPieceBytes - 1) / kPieceBytes;  // pieces of a whole chunk
+        size_t pieces = 0;
         for (size_t c = 0; c < nchunks; ++c) {
-            const size_t end = std::min(bytes, (c + 1) * chunk_bytes);
-            for (size_t o = c * chunk_bytes; o < end; o += kPieceBytes) {
-                pieces.push_back({o, std::min(kPieceBytes, end - o), c});
-                ++left[c];
-            }
+            left[c] = (uint32_t)((std::min(chunk_bytes, bytes - c * chunk_bytes) + kPieceBytes - 1) / kPieceBytes);
+            pieces += left[c];
         }
-        std::vector<hipEvent_t> done(nchunks, nullptr);
-        hipError_t err = hipSuccess;
-        for (size_t c = 0; c < nchunks && err == hipSuccess; ++c)
-            err = hipEventCreateWithFlags(&done[c], hipEventDisableTiming);
         std::mutex mu;
         std::condition_variable cv;
         std::atomic<size_t> next{0};
         std::atomic<bool> stop{false};
-        std::vector<char> ready(nchunks, 0);
         hipError_t worker_err = hipSuccess;
-        const auto work = [&](int t) {
+        auto work = [&](int t) {
             hipError_t e = hipSetDevice(set_->device);
             for (int b = 0; e == hipSuccess && !stop.load(); b ^= 1) {
                 const size_t i = next.fetch_add(1);
-                if (i >= pieces.size())
+                if (i >= pieces)
                     return;
-                const Piece &p = pieces[i];
+                const size_t c = i / per, off = c * chunk_bytes + i % per * kPieceBytes;
+                const size_t len = std::min({kPieceBytes, (c + 1) * chunk_bytes - off, bytes - off});
                 const int slot = 2 * t + b;
                 e = hipEventSynchronize(set_->ev[slot]);  // the buffer's last copy (none: at once)
                 if (e != hipSuccess)
                     break;
-                memcpy(set_->buf[slot], static_cast<const char *>(src) + p.off, p.len);
+                memcpy(set_->buf[slot], static_cast<const char *>(src) + off, len);
                 std::lock_guard<std::mutex> lock(mu);
-                e = hipMemcpyAsync(static_cast<char *>(dst) + p.off, set_->buf[slot], p.len, hipMemcpyHostToDevice,
-                                   set_->up);
+                e = hipMemcpyAsync(static_cast<char *>(dst) + off, set_->buf[slot], len, hipMemcpyHostToDevice,
+                                   set_->stream);
                 if (e == hipSuccess)
-                    e = hipEventRecord(set_->ev[slot], set_->up);
-                if (e == hipSuccess && --left[p.chunk] == 0) {
-                    e = hipEventRecord(done[p.chunk], set_->up);
-                    ready[p.chunk] = e == hipSuccess;
+                    e = hipEventRecord(set_->ev[slot], set_->stream);
+                if (e == hipSuccess && --left[c] == 0)
                     cv.notify_all();
-                }
             }
             if (e != hipSuccess) {
                 std::lock_guard<std::mutex> lock(mu);
@@ -237,46 +275,40 @@ class Staging {
                 cv.notify_all();
             }
         };
-        std::vector<std::thread> threads;
-        if (err == hipSuccess && start(threads, pieces.size(), work) > 0) {
-            ran = true;
-            for (size_t c = 0; c < nchunks && err == hipSuccess && rc == 0; ++c) {
-                {
-                    std::unique_lock<std::mutex> lock(mu);
-                    cv.wait(lock, [&] { return ready[c] || worker_err != hipSuccess; });
-                    err = worker_err;
-                }
-                if (err == hipSuccess)
-                    err = hipStreamWaitEvent(nullptr, done[c], 0);
-                if (err == hipSuccess)
-                    rc = launch(c * chunk_bytes, std::min(chunk_bytes, bytes - c * chunk_bytes));
+        set_->start(work, pieces);
+        hipError_t err = hipSuccess;
+        for (size_t c = 0; c < nchunks && err == hipSuccess && rc == 0; ++c) {
+            {
+                std::unique_lock<std::mutex> lock(mu);
+                cv.wait(lock, [&] { return left[c] == 0 || worker_err != hipSuccess; });
+                err = worker_err;
             }
-            stop = err != hipSuccess || rc != 0;
-        } else {
-            err = hipSuccess;
+            // (the marker may lie behind pieces of later chunks: a little late, never early)
+            if (err == hipSuccess)
+                err = hipEventRecord(set_->mark, set_->stream);
+            if (err == hipSuccess)
+                err = hipStreamWaitEvent(nullptr, set_->mark, 0);
+            if (err == hipSuccess)
+                rc = launch(c * chunk_bytes, std::min(chunk_bytes, bytes - c * chunk_bytes));
         }
-        for (std::thread &th : threads)
-            th.join();
-        for (hipEvent_t e : done)
-            if (e)
-                (void)hipEventDestroy(e);
+        if (err != hipSuccess || rc != 0)
+            stop = true;
+        set_->join();
         return err;
     }
 
-    hipError_t staged_download(const void *src, void *dst, size_t bytes, bool &ran) {
+    hipError_t staged_download(const void *src, void *dst, size_t bytes) {
         const size_t pieces = (bytes + kPieceBytes - 1) / kPieceBytes;
-        hipError_t err = hipEventRecord(set_->fence, nullptr);
+        hipError_t err = hipEventRecord(set_->mark, nullptr);
         if (err == hipSuccess)
-            err = hipStreamWaitEvent(set_->down, set_->fence, 0);
-        if (err != hipSuccess) {
-            ran = true;
+            err = hipStreamWaitEvent(set_->stream, set_->mark, 0);
+        if (err != hipSuccess)
             return err;
-        }
         std::mutex mu;
         std::atomic<size_t> next{0};
         std::atomic<bool> stop{false};
         hipError_t worker_err = hipSuccess;
-        const auto work = [&](int t) {
+        auto work = [&](int t) {
             hipError_t e = hipSetDevice(set_->device);
             // two pieces in turn: one on its way while the other is copied out
             size_t at[2], len[2] = {0, 0};
@@ -299,9 +331,9 @@ class Staging {
                 const size_t l = std::min(kPieceBytes, bytes - at[b]);
                 std::lock_guard<std::mutex> lock(mu);
                 e = hipMemcpyAsync(set_->buf[2 * t + b], static_cast<const char *>(src) + at[b], l,
-                                   hipMemcpyDeviceToHost, set_->down);
+                                   hipMemcpyDeviceToHost, set_->stream);
                 if (e == hipSuccess)
-                    e = hipEventRecord(set_->ev[2 * t + b], set_->down);
+                    e = hipEventRecord(set_->ev[2 * t + b], set_->stream);
                 if (e == hipSuccess)
                     len[b] = l;
             }
@@ -313,11 +345,8 @@ class Staging {
                 stop = true;
             }
         };
-        std::vector<std::thread> threads;
-        if (start(threads, pieces, work) > 0)
-            ran = true;
-        for (std::thread &th : threads)
-            th.join();
+        set_->start(work, pieces);
+        set_->join();
         return worker_err;
     }
 

@@ -7,6 +7,7 @@ distances of the returned neighbours against the FP64 optimum, to FP32 accuracy.
 """
 import ctypes
 import sys
+import threading
 import time
 
 import numpy as np
@@ -289,3 +290,105 @@ def test_settling_one_row_costs_little():
     none, one = (call_seconds(lambda v=v: ca.gpu_assign(v, c)) for v in (x, y))
     say(f"[tools] assign {n} x {dim}, k {k}: no row settled {none * 1e3:.3f} ms, one {one * 1e3:.3f} ms")
     assert one <= 1.3 * none
+
+
+def fp64_nearest(x, c):
+    """Nearest centroid of each row in FP64, and the distance to the second nearest less that."""
+    d = fp64_scores(c, x, 0)
+    two = np.partition(d, 1, axis=1)[:, :2]
+    return d.argmin(1), two[:, 1] - two[:, 0]
+
+
+def test_assign_rows_in_several_chunks():
+    """84 MB of rows: two chunks of the staged upload, the first assigned while the second is on its
+    way (their split operands and tile minima share arrays). Every row's FP64 nearest."""
+    rng = np.random.default_rng(31)
+    n, dim, k = 70_001, 300, 200
+    c = rng.standard_normal((k, dim)).astype(np.float32)
+    x = (c[rng.integers(0, k, n)] + rng.standard_normal((n, dim))).astype(np.float32)
+    say(f"[tools] assign {n} x {dim} in chunks")
+    want, gap = fp64_nearest(x, c)
+    assert gap.min() > 1e-9
+    assert np.array_equal(ca.gpu_assign(x, c), want)
+
+
+def test_kmeans_rows_in_several_chunks():
+    """The rows of some clusters lie in the second chunk of the upload alone: after one iteration
+    every centroid is the mean of the rows nearest to its first row (which no iteration returns)."""
+    rng = np.random.default_rng(32)
+    n, dim, k = 70_001, 300, 24
+    centers = 3 * rng.standard_normal((k, dim)).astype(np.float32)
+    lab = np.where(np.arange(n) < 56_000, rng.integers(0, k // 2, n), rng.integers(k // 2, k, n))
+    x = (centers[lab] + rng.standard_normal((n, dim))).astype(np.float32)
+    say(f"[tools] k-means {n} x {dim} in chunks")
+    first, c = ca.gpu_kmeans(x, k, 0, seed=1), ca.gpu_kmeans(x, k, 1, seed=1)
+    a, gap = fp64_nearest(x, first)
+    assert gap.min() > 1e-9
+    for j in range(k):
+        rows = x[a == j].astype(np.float64)
+        # m additions in any order, each rounded within 2^-24 of a partial sum of at most sum |x|
+        tol = 2.0 ** -24 * (len(rows) + 2) * np.abs(rows).mean(0).max()
+        assert np.abs(c[j] - rows.mean(0)).max() <= tol, j
+
+
+def test_rotate_rows_in_several_chunks():
+    """An upload of two chunks and a download longer than the page-locked buffers (each reused),
+    neither a whole number of 4 MiB pieces."""
+    rng = np.random.default_rng(33)
+    n, dim, P = 70_001, 300, 320
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    R = np.linalg.qr(rng.standard_normal((P, P)))[0][:dim].astype(np.float32)
+    say(f"[tools] rotate {n} x {dim} in chunks")
+    ref = x.astype(np.float64) @ R.astype(np.float64)
+    # a sum of dim products: its roundings are within dim 2^-24 of the row norms' product
+    tol = dim * 2.0 ** -24 * np.linalg.norm(x, axis=1).max()
+    assert np.abs(ca.gpu_rotate(x, R) - ref).max() < tol
+
+
+def test_quantise_rows_in_several_chunks():
+    """More than three rounds of the resident waves, with a ragged last one, uploaded and
+    downloaded through the page-locked buffers: the host's codes and factors at every row (but for
+    rows whose best t lies below the GPU sweep's start)."""
+    rng = np.random.default_rng(34)
+    n, P = 40_001, 256
+    x = rng.standard_normal((n, P)).astype(np.float32)
+    cen = 0.1 * rng.standard_normal((1, P)).astype(np.float32)
+    say(f"[tools] quantise {n} x {P} in chunks")
+    bits, f1, code, f2 = ca.quantize_rows(x, cen[0], 0)
+    R, asg = np.eye(P, dtype=np.float32), np.zeros(n, np.uint32)
+    gb, g1 = np.empty((n, P // 8), np.uint8), np.empty((n, 3), np.float32)
+    gc, g2 = np.empty((n, P), np.uint8), np.empty((n, 2), np.float32)
+    p = [a.ctypes.data_as(ctypes.c_void_p) for a in (x, R, cen, asg, gb, g1, gc, g2)]
+    assert ca.libs()[0].cora_tool_quantize(p[0], n, P, p[1], P, p[2], 1, p[3], 0, p[4], p[5], p[6], p[7], 0) == 0
+    assert np.array_equal(np.unpackbits(gb, axis=1), bits)
+    assert np.array_equal(g1.view(np.uint32), f1.view(np.uint32))
+    for r in np.nonzero((gc != code).any(1) | (g2.view(np.uint32) != f2.view(np.uint32)).any(1))[0]:
+        oa = orc.excode_residual_abs(x[r], cen[0])[1]
+        assert orc.best_rescale_factor(oa, 7) < 0.81 * 137 / float(oa.max()), r
+
+
+def test_tools_from_several_threads():
+    """Calls on different data at once, from more threads than staging sets are kept: each gets its
+    own answer."""
+    rng = np.random.default_rng(35)
+    n, dim, k = 40_000, 256, 100
+    jobs = []
+    for _ in range(4):
+        c = rng.standard_normal((k, dim)).astype(np.float32)
+        x = (c[rng.integers(0, k, n)] + rng.standard_normal((n, dim))).astype(np.float32)
+        jobs.append((x, c, fp64_nearest(x, c)[0]))
+    say("[tools] assign from four threads")
+    got = [[None] * 3 for _ in jobs]
+
+    def work(i):
+        for r in range(3):
+            got[i][r] = ca.gpu_assign(jobs[i][0], jobs[i][1])
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i, job in enumerate(jobs):
+        for r in range(3):
+            assert np.array_equal(got[i][r], job[2]), (i, r)
