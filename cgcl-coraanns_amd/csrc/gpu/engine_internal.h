@@ -325,9 +325,11 @@ void launch_split_f16_rows(const float *x, uint32_t rows, uint32_t P, uint16_t *
                            hipStream_t s);
 // the same from rows of P values to rows of Pp >= P (zeros between); norm (or nullptr): the rows'
 // squared norms
-// (copy: the rows themselves too, unless nullptr)
+// (copy: the rows themselves too, unless nullptr; shift [P]: subtracted from every row first, unless
+// nullptr)
 void launch_split_f16_padded(const float *x, uint32_t rows, uint32_t P, uint32_t Pp, uint16_t *hi, uint16_t *lo,
-                             float *scale, float *norm, hipStream_t s, float *copy = nullptr);
+                             float *scale, float *norm, hipStream_t s, float *copy = nullptr,
+                             const float *shift = nullptr);
 // an inner dimension rounded up to the split-FP16 GEMM's step
 uint32_t split_padded(uint64_t dim);
 // inner dimension K % 32 == 0 and rows * K < 2^31 for both operands

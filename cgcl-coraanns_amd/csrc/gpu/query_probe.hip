@@ -274,26 +274,28 @@ __device__ __forceinline__ int split_exponent(float amax) {
     return amax > 0.0f && amax <= FLT_MAX ? min(max(14 - ilogbf(amax), -100), 100) : 0;
 }
 
-// rows of P values to rows of Pp (zeros past P); copy: the values too (nullptr: not wanted);
-// norm: the rows' squared norms too, summed as
-// row_norms_kernel sums them (nullptr: not wanted)
+// rows of P values (less shift [P], unless nullptr) to rows of Pp (zeros past P); copy: the values
+// too (nullptr: not wanted); norm: the rows' squared norms too, summed as row_norms_kernel sums
+// them (nullptr: not wanted)
 __global__ __launch_bounds__(64) void split_f16_kernel(const float *__restrict__ x, uint32_t rows,
                                                        uint32_t P, uint32_t Pp, _Float16 *__restrict__ hi,
                                                        _Float16 *__restrict__ lo,
                                                        float *__restrict__ scale, float *__restrict__ norm,
-                                                       float *__restrict__ copy) {
+                                                       float *__restrict__ copy, const float *__restrict__ shift) {
     const int lane = threadIdx.x;
     for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x) {
         const float *row = x + (size_t)r * P;
+        const auto value = [&](uint32_t i) { return shift ? row[i] - shift[i] : row[i]; };
         float amax = 0.0f, sq = 0.0f;
         for (uint32_t i = lane; i < P; i += 64) {
-            amax = fmaxf(amax, fabsf(row[i]));
-            sq = fmaf(row[i], row[i], sq);
+            const float v = value(i);
+            amax = fmaxf(amax, fabsf(v));
+            sq = fmaf(v, v, sq);
         }
         amax = wave_max(amax);
         const int e = split_exponent(amax);
         for (uint32_t i = lane; i < Pp; i += 64) {
-            const float x0 = i < P ? row[i] : 0.0f, v = ldexpf(x0, e);
+            const float x0 = i < P ? value(i) : 0.0f, v = ldexpf(x0, e);
             if (copy && i < P)
                 copy[(size_t)r * P + i] = x0;
             const _Float16 h = (_Float16)v;
@@ -1862,11 +1864,12 @@ void launch_split_f16_rows(const float *x, uint32_t rows, uint32_t P, uint16_t *
 uint32_t split_padded(uint64_t dim) { return (uint32_t)((dim + kHK - 1) / kHK * kHK); }
 
 void launch_split_f16_padded(const float *x, uint32_t rows, uint32_t P, uint32_t Pp, uint16_t *hi, uint16_t *lo,
-                             float *scale, float *norm, hipStream_t s, float *copy) {
+                             float *scale, float *norm, hipStream_t s, float *copy, const float *shift) {
     if (!rows)
         return;
     split_f16_kernel<<<rows < (1u << 20) ? rows : (1u << 20), 64, 0, s>>>(
-        x, rows, P, Pp, reinterpret_cast<_Float16 *>(hi), reinterpret_cast<_Float16 *>(lo), scale, norm, copy);
+        x, rows, P, Pp, reinterpret_cast<_Float16 *>(hi), reinterpret_cast<_Float16 *>(lo), scale, norm, copy,
+        shift);
 }
 
 bool dist_gemm_f16x3_supported(uint32_t K, uint64_t rows_a, uint64_t rows_b) {

@@ -26,17 +26,25 @@ thread_local std::string g_tool_error;
 // ---- nearest centroid ----
 //
 // The distances ||x||^2 + ||c||^2 - 2 <x, c> come from a GEMM on split-FP16 operands, each within
-// (K + 32) 2^-24 ((||x|| + ||c||)^2) of the exact value (K products' and sums' roundings, the
-// norms' and the combination's). Where another centroid lies within the two bounds of the
-// smallest distance, the row's candidates are evaluated again in FP64 (ties -> lower id), so
+// (K + 34) 2^-24 ((||x|| + ||c||)^2) of the exact value (K products' and sums' roundings, the
+// norms' and the combination's, a shift's). Where another centroid lies within the two bounds of
+// the smallest distance, the row's candidates are evaluated again in FP64 (ties -> lower id), so
 // the answer is the FP64 one. On Gaussian mixtures that is about one row in a hundred. (The
 // FP32 GEMM's answer, where it runs instead, is its smallest distance.)
+//
+// The bound grows with the norms: rows and centroids that share an offset larger than their
+// spread are shifted by it first (nearest_shift), or every centroid would be a candidate. What
+// remains is rows far from all centroids and centroids that repeat: a row of more than
+// kNearEvals evaluations is crowded, and the crowded rows of a chunk keep the GEMM's answer (as
+// the FP32 one's, without a second look) where they would cost more than
+// kCrowdedEvals * (rows + 4096) evaluations.
+constexpr uint32_t kNearEvals = 256, kCrowdedEvals = 16;
 
 // Two bounds above the smallest computed distance: no centroid beyond it can be the nearest.
 // A candidate's norm is at most ||x|| plus its distance.
 __device__ __forceinline__ float nearest_cut(float best, float xnorm, uint32_t dim) {
     const float r = 2.0f * sqrtf(fmaxf(xnorm, 0.0f)) + sqrtf(fmaxf(best, 0.0f));
-    return best + 2.2f * (float)(dim + 32) * 0x1p-24f * r * r;
+    return best + 2.2f * (float)(dim + 34) * 0x1p-24f * r * r;
 }
 
 // argmin over each row of dist [rows][k] (FP32 GEMM); ties -> lower index.
@@ -71,38 +79,53 @@ __device__ __forceinline__ float float_of_key(uint32_t key) {
 
 // The same from the split-FP16 GEMM's smallest and second smallest distance of every 128
 // centroids (launch_nearest_gemm): a wave per row; rows with more than one candidate go to
-// list (its length in *count).
+// list [rows], crowded ones from its end (count: how many of each).
 __global__ __launch_bounds__(256) void nearest_rows_kernel(const unsigned long long *__restrict__ best,
                                                            const uint32_t *__restrict__ second, uint32_t rows,
                                                            uint32_t tiles, const float *__restrict__ xn, uint32_t dim,
                                                            uint32_t *__restrict__ out, uint32_t *__restrict__ list,
                                                            uint32_t *__restrict__ count) {
+    __shared__ uint32_t s_n[2], s_at[2];
     const uint32_t row = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63;
-    if (row >= rows)
-        return;
-    const unsigned long long *b = best + (size_t)row * tiles;
-    const uint32_t *sec = second + (size_t)row * tiles;
-    unsigned long long mine = ~0ull;
-    for (uint32_t t = lane; t < tiles; t += 64)
-        mine = min(mine, b[t]);
+    if (threadIdx.x < 2)
+        s_n[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t n = 0;  // evaluations: a tile's best, or the whole tile
+    if (row < rows) {
+        const unsigned long long *b = best + (size_t)row * tiles;
+        const uint32_t *sec = second + (size_t)row * tiles;
+        unsigned long long mine = ~0ull;
+        for (uint32_t t = lane; t < tiles; t += 64)
+            mine = min(mine, b[t]);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        mine = min(mine, (unsigned long long)__shfl_xor(mine, o, 64));
-    const float d = float_of_key((uint32_t)(mine >> 32));
-    const bool finite = (mine >> 32) < 0xFF7FFFFFull;  // below +FLT_MAX's key
-    if (lane == 0)
-        out[row] = finite ? (uint32_t)mine : 0u;
-    if (!finite)
-        return;
-    const float cut = nearest_cut(d, xn[row], dim);
-    uint32_t n = 0;
-    for (uint32_t t = lane; t < tiles; t += 64)
-        n += (float_of_key((uint32_t)(b[t] >> 32)) <= cut ? 1u : 0u) + (float_of_key(sec[t]) <= cut ? 1u : 0u);
+        for (int o = 32; o > 0; o >>= 1)
+            mine = min(mine, (unsigned long long)__shfl_xor(mine, o, 64));
+        const float d = float_of_key((uint32_t)(mine >> 32));
+        const bool finite = (mine >> 32) < 0xFF7FFFFFull;  // below +FLT_MAX's key
+        if (lane == 0)
+            out[row] = finite ? (uint32_t)mine : 0u;
+        if (finite) {
+            const float cut = nearest_cut(d, xn[row], dim);
+            for (uint32_t t = lane; t < tiles; t += 64)
+                n += float_of_key(sec[t]) <= cut ? 128u : float_of_key((uint32_t)(b[t] >> 32)) <= cut ? 1u : 0u;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        n += __shfl_xor(n, o, 64);
+            for (int o = 32; o > 0; o >>= 1)
+                n += __shfl_xor(n, o, 64);
+        }
+    }
+    // one atomic a workgroup and list: they run one after the other
+    const uint32_t which = n > kNearEvals ? 1u : 0u;
+    uint32_t at = 0;
     if (n > 1 && lane == 0)
-        list[atomicAdd(count, 1u)] = row;
+        at = atomicAdd(&s_n[which], 1u);
+    __syncthreads();
+    if (threadIdx.x < 2 && s_n[threadIdx.x])
+        s_at[threadIdx.x] = atomicAdd(&count[threadIdx.x], s_n[threadIdx.x]);
+    __syncthreads();
+    if (n > 1 && lane == 0) {
+        at += s_at[which];
+        list[which ? rows - 1 - at : at] = row;
+    }
 }
 
 // sum (x - c)^2 in FP64 for N centroids at a time by a group of eight lanes (the same in all of
@@ -154,15 +177,18 @@ __global__ __launch_bounds__(256) void nearest_exact_kernel(const unsigned long 
                                                             const float *__restrict__ x, const float *__restrict__ xn,
                                                             const float *__restrict__ cent, uint32_t k, uint32_t dim,
                                                             const uint32_t *__restrict__ list,
-                                                            const uint32_t *__restrict__ count,
+                                                            const uint32_t *__restrict__ count, uint32_t rows,
                                                             uint32_t *__restrict__ out) {
     __shared__ unsigned long long s_min[4];
     __shared__ double s_d[4];
     __shared__ uint32_t s_c[4];
     __shared__ uint32_t s_item[256], s_whole[256], s_items, s_wholes;
-    const uint32_t t = threadIdx.x, wave = t / 64, lane = t & 63, group = t / 8, gl = t & 7, n = *count;
+    const uint32_t t = threadIdx.x, wave = t / 64, lane = t & 63, group = t / 8, gl = t & 7;
+    const uint32_t near = count[0];
+    const bool crowded = (uint64_t)count[1] * k <= kCrowdedEvals * ((uint64_t)rows + 4096);
+    const uint32_t n = near + (crowded ? count[1] : 0u);
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const uint32_t row = list[i];
+        const uint32_t row = list[i < near ? i : rows - 1 - (i - near)];
         const unsigned long long *b = best + (size_t)row * tiles;
         const uint32_t *sec = second + (size_t)row * tiles;
         unsigned long long mine = ~0ull;
@@ -331,9 +357,10 @@ struct SplitRows {
         for (DevBuf *b : {&hi, &lo, &scale, &norm})
             b->release();
     }
-    void fill(const float *d_x, size_t row0, uint32_t rows, uint32_t dim, uint32_t Kp, hipStream_t s) {
+    void fill(const float *d_x, size_t row0, uint32_t rows, uint32_t dim, uint32_t Kp, hipStream_t s,
+              const float *shift = nullptr) {
         launch_split_f16_padded(d_x, rows, dim, Kp, (uint16_t *)hi.p + row0 * Kp, (uint16_t *)lo.p + row0 * Kp,
-                                (float *)scale.p + row0, (float *)norm.p + row0, s);
+                                (float *)scale.p + row0, (float *)norm.p + row0, s, nullptr, shift);
     }
 };
 
@@ -345,7 +372,8 @@ struct Nearest {
     uint32_t dim = 0, Kp = 0, k = 0, tiles = 0;
     size_t chunk = 0;
     SplitRows c;
-    DevBuf best, second, list, count;
+    DevBuf best, second, list, count, offset;
+    const float *shift = nullptr;  // subtracted from rows and centroids (device), or nullptr
     static bool supported(uint64_t dim, uint64_t k) { return k * split_padded(dim) < (1ull << 31); }
     int init(uint64_t dim_, uint64_t k_, size_t max_rows) {
         dim = (uint32_t)dim_;
@@ -355,14 +383,37 @@ struct Nearest {
         // 32-bit element offsets of a chunk's rows, and 1 GiB of tile minima
         chunk = std::max<size_t>(1, std::min<size_t>({max_rows, ((1ull << 31) - 1) / Kp, (1ull << 30) / (12ull * tiles)}));
         return c.alloc(k, Kp) || dev<unsigned long long>(best, chunk * tiles) || dev<uint32_t>(second, chunk * tiles) ||
-               dev<uint32_t>(list, chunk) || dev<uint32_t>(count, 1);
+               dev<uint32_t>(list, chunk) || dev<uint32_t>(count, 2) || dev<float>(offset, dim);
+    }
+    // The mean of up to 256 of the (host) centroids, where it is longer than their spread about it:
+    // taking away less would not make the norms much smaller.
+    int set_shift(const float *h_c) {
+        const size_t step = std::max<size_t>(1, k / 256), n = (k + step - 1) / step;
+        std::vector<double> sum(dim, 0.0);
+        double square = 0.0, offset2 = 0.0;
+        for (size_t i = 0; i < k; i += step)
+            for (uint32_t d = 0; d < dim; ++d) {
+                const double v = h_c[i * dim + d];
+                sum[d] += v;
+                square += v * v;
+            }
+        std::vector<float> mean(dim);
+        for (uint32_t d = 0; d < dim; ++d) {
+            mean[d] = (float)(sum[d] / (double)n);
+            offset2 += (double)mean[d] * mean[d];
+        }
+        if (!(offset2 > 0.5 * square / (double)n && offset2 < (double)FLT_MAX))  // nor where it is not finite
+            return CORA_OK;
+        TCHK(hipMemcpy(offset.p, mean.data(), dim * 4, hipMemcpyHostToDevice));
+        shift = (const float *)offset.p;
+        return CORA_OK;
     }
     void release() {
         c.release();
-        for (DevBuf *b : {&best, &second, &list, &count})
+        for (DevBuf *b : {&best, &second, &list, &count, &offset})
             b->release();
     }
-    void set_centroids(const float *d_c, hipStream_t s) { c.fill(d_c, 0, k, dim, Kp, s); }
+    void set_centroids(const float *d_c, hipStream_t s) { c.fill(d_c, 0, k, dim, Kp, s, shift); }
     // rows [r0, r0 + n) of x (split in xs from row s0): assign[r0 ..]
     void assign(const float *d_x, const SplitRows &xs, size_t s0, size_t n, const float *d_c, uint32_t *d_assign,
                 hipStream_t s) {
@@ -370,7 +421,7 @@ struct Nearest {
             const uint32_t rows = (uint32_t)std::min(chunk, n - b);
             const size_t at = s0 + b;
             const float *xn = (const float *)xs.norm.p + at;
-            launch_fill_u32((uint32_t *)count.p, 0u, 1, s);
+            launch_fill_u32((uint32_t *)count.p, 0u, 2, s);
             launch_nearest_gemm((const uint16_t *)xs.hi.p + at * Kp, (const uint16_t *)xs.lo.p + at * Kp,
                                 (const float *)xs.scale.p + at, xn, (const uint16_t *)c.hi.p, (const uint16_t *)c.lo.p,
                                 (const float *)c.scale.p, (const float *)c.norm.p, rows, k, Kp,
@@ -380,7 +431,7 @@ struct Nearest {
                                                                d_assign + b, (uint32_t *)list.p, (uint32_t *)count.p);
             nearest_exact_kernel<<<std::min<uint32_t>(rows, 2048), 256, 0, s>>>(
                 (const unsigned long long *)best.p, (const uint32_t *)second.p, tiles, d_x + b * dim, xn, d_c, k, dim,
-                (const uint32_t *)list.p, (const uint32_t *)count.p, d_assign + b);
+                (const uint32_t *)list.p, (const uint32_t *)count.p, rows, d_assign + b);
         }
     }
 };
@@ -559,12 +610,16 @@ int cora_tool_kmeans(const float *h_x, uint64_t n, uint64_t dim, uint64_t k, uin
     }
     if (!split && (dev<float>(cn, k) || dev<float>(xn, chunk) || dev<float>(dist, chunk * k)))
         return CORA_ERR_RUNTIME;
+    if (split)
+        if (int rc = near.set_shift(init.data()))
+            return rc;
     Staging st(device);
     int rc_copy = 0;
     TCHK(st.upload(h_x, x.p, n * dim * 4, copy_chunk_rows(dim) * dim * 4, rc_copy, [&](size_t off, size_t len) {
         const size_t r0 = off / (dim * 4);
         if (split)
-            xs.fill((float *)x.p + off / 4, r0, (uint32_t)(len / (dim * 4)), (uint32_t)dim, near.Kp, nullptr);
+            xs.fill((float *)x.p + off / 4, r0, (uint32_t)(len / (dim * 4)), (uint32_t)dim, near.Kp, nullptr,
+                    near.shift);
         return 0;
     }));
     TCHK(hipMemcpy(c.p, init.data(), k * dim * 4, hipMemcpyHostToDevice));
@@ -622,9 +677,11 @@ int cora_tool_assign(const float *h_x, uint64_t n, uint64_t dim, const float *h_
     if (!split && (dev<float>(cn, k) || dev<float>(xn, chunk) || dev<float>(dist, chunk * k)))
         return CORA_ERR_RUNTIME;
     TCHK(hipMemcpy(c.p, h_centroids, k * dim * 4, hipMemcpyHostToDevice));
-    if (split)
+    if (split) {
+        if (int rc = near.set_shift(h_centroids))
+            return rc;
         near.set_centroids((float *)c.p, nullptr);
-    else
+    } else
         launch_row_norms((float *)c.p, (uint32_t)k, (uint32_t)dim, (float *)cn.p, nullptr);
     Staging st(device);
     for (size_t b = 0; b < n; b += rows_dev) {
@@ -637,7 +694,7 @@ int cora_tool_assign(const float *h_x, uint64_t n, uint64_t dim, const float *h_
             if (!split)
                 return assign_rows(xc, m, (uint32_t)dim, (float *)c.p, (float *)cn.p, (uint32_t)k, ac, (float *)xn.p,
                                    (float *)dist.p, chunk, nullptr);
-            xs.fill(xc, 0, (uint32_t)m, (uint32_t)dim, near.Kp, nullptr);
+            xs.fill(xc, 0, (uint32_t)m, (uint32_t)dim, near.Kp, nullptr, near.shift);
             near.assign(xc, xs, 0, m, (float *)c.p, ac, nullptr);
             return (int)CORA_OK;
         }));

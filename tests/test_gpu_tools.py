@@ -392,3 +392,36 @@ def test_tools_from_several_threads():
     for i, job in enumerate(jobs):
         for r in range(3):
             assert np.array_equal(got[i][r], job[2]), (i, r)
+
+
+@pytest.mark.parametrize("kind", ["offset", "repeated", "far rows"])
+def test_settling_many_rows_is_bounded(kind):
+    """Data on which the bound of a row's distances spans many centroids: a common offset of 100
+    times the spread (shifted away: the FP64 answer at every row), every centroid 64 times (the
+    first of equals), rows far away from all centroids. A call takes at most a few times the
+    time that it takes on centred data."""
+    rng = np.random.default_rng(91)
+    n, dim, k = 60_000, 128, 2048
+    c = rng.standard_normal((k, dim)).astype(np.float32)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    centred = call_seconds(lambda: ca.gpu_assign(x, c), 5)
+    if kind == "offset":
+        x, c = x + np.float32(100), c + np.float32(100)
+    elif kind == "repeated":
+        c = np.ascontiguousarray(np.tile(c[:32], (64, 1)))
+    else:
+        x *= np.float32(3e3)
+    a = ca.gpu_assign(x, c).astype(np.int64)
+    m = c.astype(np.float64).mean(0)
+    d = fp64_scores(c.astype(np.float64) - m, x.astype(np.float64) - m, 0)
+    got, best = np.take_along_axis(d, a[:, None], 1)[:, 0], d.min(1)
+    scale = (np.sqrt((x.astype(np.float64) ** 2).sum(1)) + np.sqrt(best)) ** 2
+    if kind == "offset":
+        assert np.array_equal(a, d.argmin(1))
+    elif kind == "repeated":
+        assert a.max() < 32 and np.array_equal(a, d[:, :32].argmin(1))
+    # at worst the GEMM's answer: two of its error bounds
+    assert np.all(got - best <= 2.2 * (dim + 34) * 2.0 ** -24 * scale)
+    t = call_seconds(lambda: ca.gpu_assign(x, c), 5)
+    say(f"[tools] assign {n} x {dim}, k {k}: centred {centred * 1e3:.2f} ms, {kind} {t * 1e3:.2f} ms")
+    assert t <= 3 * centred
