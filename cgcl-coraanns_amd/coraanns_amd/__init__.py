@@ -173,6 +173,7 @@ GPU_SIGNATURES = {
     "cora_gpu_debug_read": [_P, _I, _P, _U64],
     "cora_gpu_debug_dense": [_P, _P, _P, _P, _U64],
     "cora_tool_last_error": [],
+    "cora_tool_debug_no_split": [_I],
     "cora_tool_rotate": [_P, _U64, _U64, _P, _U64, _P, _I],
     "cora_tool_quantize": [_P, _U64, _U64, _P, _U64, _P, _U64, _P, _I, _P, _P, _P, _P, _I],
     "cora_tool_kmeans": [_P, _U64, _U64, _U64, C.c_uint32, _U64, _P, _I],

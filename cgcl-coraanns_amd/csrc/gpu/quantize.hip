@@ -36,6 +36,7 @@
 #include <string>
 
 #include "../../../include/cora_gpu.h"
+#include "dev_block.h"
 #include "engine_internal.h"
 #include "host_copy.h"
 
@@ -725,14 +726,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RMAX > 12 ? 
     }
 }
 
-struct QzBuf {
-    void *p = nullptr;
-    ~QzBuf() {
-        if (p)
-            (void)hipFree(p);
-    }
-};
-
 #define QCHK(call)                                                                  \
     do {                                                                            \
         hipError_t e_ = (call);                                                     \
@@ -764,18 +757,22 @@ int cora_tool_quantize(const float *h_x, uint64_t n, uint64_t dim, const float *
         }
     QCHK(hipSetDevice(device));
     const size_t chunk = std::min<size_t>(n, (size_t)1 << 20);
-    QzBuf x, r, xr, c, asg, bits, f1, code, f2;
-    QCHK(hipMalloc(&x.p, chunk * dim * 4));
-    QCHK(hipMalloc(&r.p, dim * P * 4));
-    QCHK(hipMalloc(&xr.p, chunk * P * 4));
-    QCHK(hipMalloc(&c.p, nlist * P * 4));
-    QCHK(hipMalloc(&asg.p, chunk * 4));
-    QCHK(hipMalloc(&bits.p, chunk * P / 8));
-    QCHK(hipMalloc(&f1.p, chunk * 12));
-    QCHK(hipMalloc(&code.p, chunk * P));
-    QCHK(hipMalloc(&f2.p, chunk * 8));
-    QCHK(hipMemcpy(r.p, h_R, dim * P * 4, hipMemcpyHostToDevice));
-    QCHK(hipMemcpy(c.p, h_centroids, nlist * P * 4, hipMemcpyHostToDevice));
+    DevBlock block;
+    float *x, *r, *xr, *c, *f1, *f2;
+    uint32_t *asg;
+    uint8_t *bits, *code;
+    block.add(x, chunk * dim);
+    block.add(r, dim * P);
+    block.add(xr, chunk * P);
+    block.add(c, nlist * P);
+    block.add(asg, chunk);
+    block.add(bits, chunk * P / 8);
+    block.add(f1, chunk * 3);
+    block.add(code, chunk * P);
+    block.add(f2, chunk * 2);
+    QCHK(block.alloc());
+    QCHK(hipMemcpy(r, h_R, dim * P * 4, hipMemcpyHostToDevice));
+    QCHK(hipMemcpy(c, h_centroids, nlist * P * 4, hipMemcpyHostToDevice));
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
     auto *kernel = P <= 128   ? quantize_kernel<2>
@@ -792,24 +789,22 @@ int cora_tool_quantize(const float *h_x, uint64_t n, uint64_t dim, const float *
     Staging st(device);
     for (size_t b = 0; b < n; b += chunk) {
         const size_t rows = std::min(chunk, (size_t)n - b);
-        QCHK(hipMemcpy(asg.p, h_assign + b, rows * 4, hipMemcpyHostToDevice));
+        QCHK(hipMemcpy(asg, h_assign + b, rows * 4, hipMemcpyHostToDevice));
         int rc = 0;
-        QCHK(st.upload(h_x + b * dim, x.p, rows * dim * 4, step * dim * 4, rc, [&](size_t off, size_t len) {
+        QCHK(st.upload(h_x + b * dim, x, rows * dim * 4, step * dim * 4, rc, [&](size_t off, size_t len) {
             const size_t r0 = off / (dim * 4), m = len / (dim * 4);
-            float *out = (float *)xr.p + r0 * P;
-            launch_rotate((float *)x.p + r0 * dim, (float *)r.p, out, (uint32_t)m, (uint32_t)dim, (uint32_t)P, nullptr);
-            QzArgs qa{out,        (const float *)c.p,       (const uint32_t *)asg.p + r0,
-                      (uint32_t)m, (uint32_t)P,             metric,
-                      (uint8_t *)bits.p + r0 * (P / 8),     (float *)f1.p + r0 * 3,
-                      (uint8_t *)code.p + r0 * P,           (float *)f2.p + r0 * 2};
+            float *out = xr + r0 * P;
+            launch_rotate(x + r0 * dim, r, out, (uint32_t)m, (uint32_t)dim, (uint32_t)P, nullptr);
+            QzArgs qa{out,    c,  asg + r0, (uint32_t)m, (uint32_t)P, metric, bits + r0 * (P / 8), f1 + r0 * 3,
+                      code + r0 * P, f2 + r0 * 2};
             kernel<<<(uint32_t)std::min<size_t>(m, waves), 64>>>(qa);
             return 0;
         }));
         QCHK(hipGetLastError());
-        QCHK(st.download(bits.p, h_bits + b * (P / 8), rows * (P / 8)));
-        QCHK(st.download(f1.p, h_f1 + b * 3, rows * 12));
-        QCHK(st.download(code.p, h_code + b * P, rows * P));
-        QCHK(st.download(f2.p, h_f2 + b * 2, rows * 8));
+        QCHK(st.download(bits, h_bits + b * (P / 8), rows * (P / 8)));
+        QCHK(st.download(f1, h_f1 + b * 3, rows * 12));
+        QCHK(st.download(code, h_code + b * P, rows * P));
+        QCHK(st.download(f2, h_f2 + b * 2, rows * 8));
     }
     return CORA_OK;
 }

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../../include/cora_gpu.h"
+#include "dev_block.h"
 #include "engine_internal.h"
 #include "host_copy.h"
 
@@ -25,20 +26,20 @@ thread_local std::string g_tool_error;
 
 // ---- nearest centroid ----
 //
-// The distances ||x||^2 + ||c||^2 - 2 <x, c> come from a GEMM on split-FP16 operands, each within
-// (K + 34) 2^-24 ((||x|| + ||c||)^2) of the exact value (K products' and sums' roundings, the
-// norms' and the combination's, a shift's). Where another centroid lies within the two bounds of
-// the smallest distance, the row's candidates are evaluated again in FP64 (ties -> lower id), so
-// the answer is the FP64 one. On Gaussian mixtures that is about one row in a hundred. (The
-// FP32 GEMM's answer, where it runs instead, is its smallest distance.)
+// The distances ||x||^2 + ||c||^2 - 2 <x, c> come from a GEMM, in FP32 or on split-FP16 operands,
+// each within (K + 34) 2^-24 ((||x|| + ||c||)^2) of the exact value (K products' and sums'
+// roundings, the norms' and the combination's, a shift's). Where another centroid lies within
+// the two bounds of the smallest distance, the row's candidates are evaluated again in FP64
+// (ties -> lower id), so the answer is the FP64 one whichever GEMM ran. On Gaussian mixtures that
+// is about one row in a hundred.
 //
-// The bound grows with the norms: rows and centroids that share an offset larger than their
-// spread are shifted by it first (nearest_shift), or every centroid would be a candidate. What
-// remains is rows far from all centroids and centroids that repeat: a row of more than
-// kNearEvals evaluations is crowded, and the crowded rows of a chunk keep the GEMM's answer (as
-// the FP32 one's, without a second look) where they would cost more than
-// kCrowdedEvals * (rows + 4096) evaluations.
-constexpr uint32_t kNearEvals = 256, kCrowdedEvals = 16;
+// The bound grows with the norms. For the split GEMM, rows and centroids that share an offset
+// larger than their spread are shifted by it first (set_shift), or every centroid would be a
+// candidate. What remains is rows far from all centroids and centroids that repeat: a row of
+// more than kNearEvals evaluations is crowded, and the crowded rows of a chunk keep the GEMM's
+// answer, its smallest distance, where they would cost more than kCrowdedEvals * (rows + 4096)
+// evaluations. After the FP32 GEMM a row of more than kNearFew candidates keeps it.
+constexpr uint32_t kNearEvals = 256, kCrowdedEvals = 16, kNearFew = 16;
 
 // Two bounds above the smallest computed distance: no centroid beyond it can be the nearest.
 // A candidate's norm is at most ||x|| plus its distance.
@@ -47,29 +48,114 @@ __device__ __forceinline__ float nearest_cut(float best, float xnorm, uint32_t d
     return best + 2.2f * (float)(dim + 34) * 0x1p-24f * r * r;
 }
 
-// argmin over each row of dist [rows][k] (FP32 GEMM); ties -> lower index.
+// sum (x - c)^2 in FP64 for N centroids at a time by a group of eight lanes (the same in all of
+// them). Aligned rows of whole quads are read four values at a time.
+template <int N>
+__device__ __forceinline__ void group_l2(const float *__restrict__ x, const float *const (&c)[N], uint32_t dim,
+                                         uint32_t gl, double (&s)[N]) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        s[j] = 0.0;
+    const auto term = [](float a, float b, double acc) {
+        const double d = (double)a - (double)b;
+        return fma(d, d, acc);
+    };
+    if (dim % 4 == 0) {
+        for (uint32_t i = 4 * gl; i < dim; i += 32) {
+            const float4 a = *reinterpret_cast<const float4 *>(x + i);
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const float4 b = *reinterpret_cast<const float4 *>(c[j] + i);
+                s[j] = term(a.x, b.x, s[j]);
+                s[j] = term(a.y, b.y, s[j]);
+                s[j] = term(a.z, b.z, s[j]);
+                s[j] = term(a.w, b.w, s[j]);
+            }
+        }
+    } else {
+        for (uint32_t i = gl; i < dim; i += 8) {
+            const float a = x[i];
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+                s[j] = term(a, c[j][i], s[j]);
+        }
+    }
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            s[j] += __shfl_xor(s[j], o, 64);
+}
+
+// argmin over each row of dist [rows][k] (FP32 GEMM); ties -> lower index. A second pass over the
+// row lists its candidates where there is another; more than kNearFew are crowded.
 __global__ __launch_bounds__(64) void row_argmin_kernel(const float *__restrict__ dist, uint32_t k,
+                                                        const float *__restrict__ x, const float *__restrict__ xn,
+                                                        const float *__restrict__ cent, uint32_t dim,
                                                         uint32_t *__restrict__ out) {
+    __shared__ uint32_t s_cand[kNearFew];
     const float *row = dist + (size_t)blockIdx.x * k;
-    float best = FLT_MAX;
+    const uint32_t lane = threadIdx.x;
+    float best = FLT_MAX, next = FLT_MAX;
     uint32_t bi = 0xFFFFFFFFu;
-    for (uint32_t j = threadIdx.x; j < k; j += 64) {
+    for (uint32_t j = lane; j < k; j += 64) {
         const float v = row[j];
         if (v < best || (v == best && j < bi)) {
+            next = best;
             best = v;
             bi = j;
+        } else {
+            next = fminf(next, v);
         }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(best, o, 64);
+        const float ov = __shfl_xor(best, o, 64), on = __shfl_xor(next, o, 64);
         const uint32_t oi = __shfl_xor(bi, o, 64);
-        if (ov < best || (ov == best && oi < bi)) {
+        const bool take = ov < best || (ov == best && oi < bi);
+        next = fminf(fminf(next, on), take ? best : ov);
+        if (take) {
             best = ov;
             bi = oi;
         }
     }
-    if (threadIdx.x == 0)
+    if (bi != 0xFFFFFFFFu) {
+        const float cut = nearest_cut(best, xn[blockIdx.x], dim);
+        uint32_t n = 0;
+        for (uint32_t j0 = 0; next <= cut && j0 < k && n <= kNearFew; j0 += 64) {
+            const uint32_t j = j0 + lane;
+            const bool in = j < k && row[j] <= cut;
+            const unsigned long long m = __ballot(in);
+            const uint32_t at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            if (in && at < kNearFew)
+                s_cand[at] = j;
+            n += (uint32_t)__popcll(m);
+        }
+        __syncthreads();
+        if (n > 1 && n <= kNearFew) {
+            double bd = __longlong_as_double(0x7FF0000000000000ll);
+            for (uint32_t i = lane / 8; i < n; i += 8) {
+                const float *const c[1] = {cent + (size_t)s_cand[i] * dim};
+                double d[1];
+                group_l2<1>(x + (size_t)blockIdx.x * dim, c, dim, lane & 7, d);
+                if (i < 8 || d[0] < bd || (d[0] == bd && s_cand[i] < bi)) {
+                    bd = d[0];
+                    bi = s_cand[i];
+                }
+            }
+#pragma unroll
+            for (int o = 32; o >= 8; o >>= 1) {
+                const double od = __shfl_xor(bd, o, 64);
+                const uint32_t oi = __shfl_xor(bi, o, 64);
+                if (od < bd || (od == bd && oi < bi)) {
+                    bd = od;
+                    bi = oi;
+                }
+            }
+        }
+    }
+    if (lane == 0)
         out[blockIdx.x] = bi == 0xFFFFFFFFu ? 0u : bi;
 }
 
@@ -126,45 +212,6 @@ __global__ __launch_bounds__(256) void nearest_rows_kernel(const unsigned long l
         at += s_at[which];
         list[which ? rows - 1 - at : at] = row;
     }
-}
-
-// sum (x - c)^2 in FP64 for N centroids at a time by a group of eight lanes (the same in all of
-// them). Aligned rows of whole quads are read four values at a time.
-template <int N>
-__device__ __forceinline__ void group_l2(const float *__restrict__ x, const float *const (&c)[N], uint32_t dim,
-                                         uint32_t gl, double (&s)[N]) {
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-        s[j] = 0.0;
-    const auto term = [](float a, float b, double acc) {
-        const double d = (double)a - (double)b;
-        return fma(d, d, acc);
-    };
-    if (dim % 4 == 0) {
-        for (uint32_t i = 4 * gl; i < dim; i += 32) {
-            const float4 a = *reinterpret_cast<const float4 *>(x + i);
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const float4 b = *reinterpret_cast<const float4 *>(c[j] + i);
-                s[j] = term(a.x, b.x, s[j]);
-                s[j] = term(a.y, b.y, s[j]);
-                s[j] = term(a.z, b.z, s[j]);
-                s[j] = term(a.w, b.w, s[j]);
-            }
-        }
-    } else {
-        for (uint32_t i = gl; i < dim; i += 8) {
-            const float a = x[i];
-#pragma unroll
-            for (int j = 0; j < N; ++j)
-                s[j] = term(a, c[j][i], s[j]);
-        }
-    }
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1)
-#pragma unroll
-        for (int j = 0; j < N; ++j)
-            s[j] += __shfl_xor(s[j], o, 64);
 }
 
 // The listed rows' nearest centroid in FP64 over the candidates: a tile's best, or all 128
@@ -305,16 +352,6 @@ __global__ void gather_block_topk_kernel(const float *__restrict__ dist, uint32_
     ci[r * stride + slot0 + j] = base0 + i;
 }
 
-struct DevBuf {
-    void *p = nullptr;
-    ~DevBuf() { release(); }
-    void release() {
-        if (p)
-            (void)hipFree(p);
-        p = nullptr;
-    }
-};
-
 #define TCHK(call)                                                                  \
     do {                                                                            \
         hipError_t e_ = (call);                                                     \
@@ -323,12 +360,6 @@ struct DevBuf {
             return CORA_ERR_RUNTIME;                                                \
         }                                                                           \
     } while (0)
-
-template <class T>
-int dev(DevBuf &b, size_t n) {
-    TCHK(hipMalloc(&b.p, std::max<size_t>(1, n) * sizeof(T)));
-    return CORA_OK;
-}
 
 // Assign rows [0, n) of device matrix x to the nearest of k device centroids (FP32 GEMM, the
 // distances in d_dist [chunk][k]).
@@ -339,7 +370,7 @@ int assign_rows(const float *d_x, size_t n, uint32_t dim, const float *d_c, cons
         const uint32_t rows = (uint32_t)std::min(chunk, n - b);
         launch_row_norms(d_x + b * dim, rows, dim, d_xn, s);
         launch_dist_gemm(d_x + b * dim, d_xn, d_c, d_cn, rows, k, dim, d_dist, s);
-        row_argmin_kernel<<<rows, 64, 0, s>>>(d_dist, k, d_assign + b);
+        row_argmin_kernel<<<rows, 64, 0, s>>>(d_dist, k, d_x + b * dim, d_xn, d_c, dim, d_assign + b);
     }
     TCHK(hipGetLastError());
     return CORA_OK;
@@ -348,19 +379,18 @@ int assign_rows(const float *d_x, size_t n, uint32_t dim, const float *d_c, cons
 // Rows or centroids as split-FP16 operands: [rows][Kp] hi and lo halves (Kp: the dimension
 // rounded up to the GEMM's step), scales and squared norms.
 struct SplitRows {
-    DevBuf hi, lo, scale, norm;
-    int alloc(size_t rows, size_t Kp) {
-        return dev<uint16_t>(hi, rows * Kp) || dev<uint16_t>(lo, rows * Kp) || dev<float>(scale, rows) ||
-               dev<float>(norm, rows);
-    }
-    void release() {
-        for (DevBuf *b : {&hi, &lo, &scale, &norm})
-            b->release();
+    uint16_t *hi, *lo;
+    float *scale, *norm;
+    void add_to(DevBlock &block, size_t rows, size_t Kp) {
+        block.add(hi, rows * Kp);
+        block.add(lo, rows * Kp);
+        block.add(scale, rows);
+        block.add(norm, rows);
     }
     void fill(const float *d_x, size_t row0, uint32_t rows, uint32_t dim, uint32_t Kp, hipStream_t s,
               const float *shift = nullptr) {
-        launch_split_f16_padded(d_x, rows, dim, Kp, (uint16_t *)hi.p + row0 * Kp, (uint16_t *)lo.p + row0 * Kp,
-                                (float *)scale.p + row0, (float *)norm.p + row0, s, nullptr, shift);
+        launch_split_f16_padded(d_x, rows, dim, Kp, hi + row0 * Kp, lo + row0 * Kp, scale + row0, norm + row0, s,
+                                nullptr, shift);
     }
 };
 
@@ -372,18 +402,24 @@ struct Nearest {
     uint32_t dim = 0, Kp = 0, k = 0, tiles = 0;
     size_t chunk = 0;
     SplitRows c;
-    DevBuf best, second, list, count, offset;
+    unsigned long long *best;
+    uint32_t *second, *list, *count;
+    float *offset;
     const float *shift = nullptr;  // subtracted from rows and centroids (device), or nullptr
     static bool supported(uint64_t dim, uint64_t k) { return k * split_padded(dim) < (1ull << 31); }
-    int init(uint64_t dim_, uint64_t k_, size_t max_rows) {
+    void init(DevBlock &block, uint64_t dim_, uint64_t k_, size_t max_rows) {
         dim = (uint32_t)dim_;
         k = (uint32_t)k_;
         Kp = split_padded(dim_);
         tiles = nearest_tiles(k);
         // 32-bit element offsets of a chunk's rows, and 1 GiB of tile minima
         chunk = std::max<size_t>(1, std::min<size_t>({max_rows, ((1ull << 31) - 1) / Kp, (1ull << 30) / (12ull * tiles)}));
-        return c.alloc(k, Kp) || dev<unsigned long long>(best, chunk * tiles) || dev<uint32_t>(second, chunk * tiles) ||
-               dev<uint32_t>(list, chunk) || dev<uint32_t>(count, 2) || dev<float>(offset, dim);
+        c.add_to(block, k, Kp);
+        block.add(best, chunk * tiles);
+        block.add(second, chunk * tiles);
+        block.add(list, chunk);
+        block.add(count, 2);
+        block.add(offset, dim);
     }
     // The mean of up to 256 of the (host) centroids, where it is longer than their spread about it:
     // taking away less would not make the norms much smaller.
@@ -404,14 +440,9 @@ struct Nearest {
         }
         if (!(offset2 > 0.5 * square / (double)n && offset2 < (double)FLT_MAX))  // nor where it is not finite
             return CORA_OK;
-        TCHK(hipMemcpy(offset.p, mean.data(), dim * 4, hipMemcpyHostToDevice));
-        shift = (const float *)offset.p;
+        TCHK(hipMemcpy(offset, mean.data(), dim * 4, hipMemcpyHostToDevice));
+        shift = offset;
         return CORA_OK;
-    }
-    void release() {
-        c.release();
-        for (DevBuf *b : {&best, &second, &list, &count, &offset})
-            b->release();
     }
     void set_centroids(const float *d_c, hipStream_t s) { c.fill(d_c, 0, k, dim, Kp, s, shift); }
     // rows [r0, r0 + n) of x (split in xs from row s0): assign[r0 ..]
@@ -420,31 +451,30 @@ struct Nearest {
         for (size_t b = 0; b < n; b += chunk) {
             const uint32_t rows = (uint32_t)std::min(chunk, n - b);
             const size_t at = s0 + b;
-            const float *xn = (const float *)xs.norm.p + at;
-            launch_fill_u32((uint32_t *)count.p, 0u, 2, s);
-            launch_nearest_gemm((const uint16_t *)xs.hi.p + at * Kp, (const uint16_t *)xs.lo.p + at * Kp,
-                                (const float *)xs.scale.p + at, xn, (const uint16_t *)c.hi.p, (const uint16_t *)c.lo.p,
-                                (const float *)c.scale.p, (const float *)c.norm.p, rows, k, Kp,
-                                (unsigned long long *)best.p, (uint32_t *)second.p, s);
-            nearest_rows_kernel<<<(rows + 3) / 4, 256, 0, s>>>((const unsigned long long *)best.p,
-                                                               (const uint32_t *)second.p, rows, tiles, xn, dim,
-                                                               d_assign + b, (uint32_t *)list.p, (uint32_t *)count.p);
-            nearest_exact_kernel<<<std::min<uint32_t>(rows, 2048), 256, 0, s>>>(
-                (const unsigned long long *)best.p, (const uint32_t *)second.p, tiles, d_x + b * dim, xn, d_c, k, dim,
-                (const uint32_t *)list.p, (const uint32_t *)count.p, rows, d_assign + b);
+            const float *xn = xs.norm + at;
+            launch_fill_u32(count, 0u, 2, s);
+            launch_nearest_gemm(xs.hi + at * Kp, xs.lo + at * Kp, xs.scale + at, xn, c.hi, c.lo, c.scale, c.norm, rows,
+                                k, Kp, best, second, s);
+            nearest_rows_kernel<<<(rows + 3) / 4, 256, 0, s>>>(best, second, rows, tiles, xn, dim, d_assign + b, list,
+                                                               count);
+            nearest_exact_kernel<<<std::min<uint32_t>(rows, 2048), 256, 0, s>>>(best, second, tiles, d_x + b * dim, xn,
+                                                                                d_c, k, dim, list, count, rows,
+                                                                                d_assign + b);
         }
     }
 };
 
 // The split operands of whole arrays take as much device memory again as the arrays. Where it is
-// not there (ok: they were allocated), the call goes on without them, on the FP32 GEMM, which
-// reads the rows as they are: what fitted the device before still does.
-bool split_or_fp32(bool ok) {
-    if (!ok) {
-        (void)hipGetLastError();
-        g_tool_error.clear();
-    }
-    return ok;
+// not there, the call goes on without them, on the FP32 GEMM, which reads the rows as they are:
+// what fitted the device before still does.
+thread_local bool g_no_split = false;  // cora_tool_debug_no_split
+bool split_or_fp32(DevBlock &split) {
+    if (g_no_split)
+        return false;
+    if (split.alloc() == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 // rows of a chunk that is computed on while the next ones are copied: whole GEMM tiles, 64 MiB
@@ -499,30 +529,37 @@ extern "C" {
 
 const char *cora_tool_last_error(void) { return g_tool_error.c_str(); }
 
+int cora_tool_debug_no_split(int on) {
+    const int was = g_no_split;
+    g_no_split = on != 0;
+    return was;
+}
+
 int cora_tool_rotate(const float *h_x, uint64_t n, uint64_t dim, const float *h_R, uint64_t P,
                      float *h_out, int device) {
     if (!h_x || !h_R || !h_out || !n || !dim || P < dim)
         return CORA_ERR_INVALID_ARGUMENT;
     TCHK(hipSetDevice(device));
-    DevBuf x, r, o;
     const size_t chunk = 1u << 20;
-    if (dev<float>(x, std::min<size_t>(n, chunk) * dim) || dev<float>(r, dim * P) ||
-        dev<float>(o, std::min<size_t>(n, chunk) * P))
-        return CORA_ERR_RUNTIME;
+    DevBlock block;
+    float *x, *r, *o;
+    block.add(x, std::min<size_t>(n, chunk) * dim);
+    block.add(r, dim * P);
+    block.add(o, std::min<size_t>(n, chunk) * P);
+    TCHK(block.alloc());
     Staging st(device);
-    TCHK(hipMemcpy(r.p, h_R, dim * P * 4, hipMemcpyHostToDevice));
+    TCHK(hipMemcpy(r, h_R, dim * P * 4, hipMemcpyHostToDevice));
     for (size_t b = 0; b < n; b += chunk) {
         const size_t rows = std::min<size_t>(chunk, n - b);
         int rc = 0;
-        TCHK(st.upload(h_x + b * dim, x.p, rows * dim * 4, copy_chunk_rows(dim) * dim * 4, rc,
+        TCHK(st.upload(h_x + b * dim, x, rows * dim * 4, copy_chunk_rows(dim) * dim * 4, rc,
                        [&](size_t off, size_t len) {
                            const size_t r0 = off / (dim * 4), m = len / (dim * 4);
-                           launch_rotate((float *)x.p + r0 * dim, (float *)r.p, (float *)o.p + r0 * P, (uint32_t)m,
-                                         (uint32_t)dim, (uint32_t)P, nullptr);
+                           launch_rotate(x + r0 * dim, r, o + r0 * P, (uint32_t)m, (uint32_t)dim, (uint32_t)P, nullptr);
                            return 0;
                        }));
         TCHK(hipGetLastError());
-        TCHK(st.download(o.p, h_out + b * P, rows * P * 4));  // the rows are read before the next ones come
+        TCHK(st.download(o, h_out + b * P, rows * P * 4));  // the rows are read before the next ones come
     }
     return CORA_OK;
 }
@@ -598,61 +635,71 @@ int cora_tool_kmeans(const float *h_x, uint64_t n, uint64_t dim, uint64_t k, uin
         memcpy(&init[i * dim], h_x + pick[i] * dim, dim * 4);
     bool split = Nearest::supported(dim, k);
     const size_t chunk = std::max<size_t>(1, std::min<size_t>(n, (size_t)(1u << 30) / (k * 4)));
-    DevBuf x, c, cn, xn, dist, asg, sums, cnt;
+    DevBlock block, split_block, fp32_block;
+    float *x, *c, *sums, *cn, *xn, *dist;
+    uint32_t *asg, *cnt;
     Nearest near;
     SplitRows xs;
-    if (dev<float>(x, n * dim) || dev<float>(c, k * dim) || dev<uint32_t>(asg, n) ||
-        dev<float>(sums, k * dim) || dev<uint32_t>(cnt, k))
-        return CORA_ERR_RUNTIME;
-    if (split && !(split = split_or_fp32(!near.init(dim, k, n) && !xs.alloc(n, near.Kp)))) {
-        near.release();
-        xs.release();
+    block.add(x, n * dim);
+    block.add(c, k * dim);
+    block.add(asg, n);
+    block.add(sums, k * dim);
+    block.add(cnt, k);
+    TCHK(block.alloc());
+    if (split) {
+        near.init(split_block, dim, k, n);
+        xs.add_to(split_block, n, near.Kp);
+        split = split_or_fp32(split_block);
     }
-    if (!split && (dev<float>(cn, k) || dev<float>(xn, chunk) || dev<float>(dist, chunk * k)))
-        return CORA_ERR_RUNTIME;
+    if (!split) {
+        fp32_block.add(cn, k);
+        fp32_block.add(xn, chunk);
+        fp32_block.add(dist, chunk * k);
+        TCHK(fp32_block.alloc());
+    }
     if (split)
         if (int rc = near.set_shift(init.data()))
             return rc;
     Staging st(device);
     int rc_copy = 0;
-    TCHK(st.upload(h_x, x.p, n * dim * 4, copy_chunk_rows(dim) * dim * 4, rc_copy, [&](size_t off, size_t len) {
+    TCHK(st.upload(h_x, x, n * dim * 4, copy_chunk_rows(dim) * dim * 4, rc_copy, [&](size_t off, size_t len) {
         const size_t r0 = off / (dim * 4);
         if (split)
-            xs.fill((float *)x.p + off / 4, r0, (uint32_t)(len / (dim * 4)), (uint32_t)dim, near.Kp, nullptr,
+            xs.fill(x + off / 4, r0, (uint32_t)(len / (dim * 4)), (uint32_t)dim, near.Kp, nullptr,
                     near.shift);
         return 0;
     }));
-    TCHK(hipMemcpy(c.p, init.data(), k * dim * 4, hipMemcpyHostToDevice));
+    TCHK(hipMemcpy(c, init.data(), k * dim * 4, hipMemcpyHostToDevice));
     std::vector<uint32_t> counts(k);
     std::mt19937_64 split_gen(seed ^ 0x9E3779B97F4A7C15ull);
     for (uint32_t it = 0; it < iters; ++it) {
         if (split) {
-            near.set_centroids((float *)c.p, nullptr);
-            near.assign((float *)x.p, xs, 0, n, (float *)c.p, (uint32_t *)asg.p, nullptr);
+            near.set_centroids(c, nullptr);
+            near.assign(x, xs, 0, n, c, asg, nullptr);
         } else {
-            launch_row_norms((float *)c.p, (uint32_t)k, (uint32_t)dim, (float *)cn.p, nullptr);
-            if (int rc = assign_rows((float *)x.p, n, (uint32_t)dim, (float *)c.p, (float *)cn.p,
-                                     (uint32_t)k, (uint32_t *)asg.p, (float *)xn.p, (float *)dist.p,
+            launch_row_norms(c, (uint32_t)k, (uint32_t)dim, cn, nullptr);
+            if (int rc = assign_rows(x, n, (uint32_t)dim, c, cn,
+                                     (uint32_t)k, asg, xn, dist,
                                      chunk, nullptr))
                 return rc;
         }
-        TCHK(hipMemset(sums.p, 0, k * dim * 4));
-        TCHK(hipMemset(cnt.p, 0, k * 4));
-        accumulate_kernel<<<(uint32_t)std::min<uint64_t>(n, 1u << 20), 64>>>((float *)x.p, (uint32_t *)asg.p, (uint32_t)n,
-                                                (uint32_t)dim, (float *)sums.p, (uint32_t *)cnt.p);
-        update_kernel<<<(uint32_t)((k * dim + 255) / 256), 256>>>((float *)c.p, (float *)sums.p,
-                                                                   (uint32_t *)cnt.p, (uint32_t)k,
+        TCHK(hipMemset(sums, 0, k * dim * 4));
+        TCHK(hipMemset(cnt, 0, k * 4));
+        accumulate_kernel<<<(uint32_t)std::min<uint64_t>(n, 1u << 20), 64>>>(x, asg, (uint32_t)n,
+                                                (uint32_t)dim, sums, cnt);
+        update_kernel<<<(uint32_t)((k * dim + 255) / 256), 256>>>(c, sums,
+                                                                   cnt, (uint32_t)k,
                                                                    (uint32_t)dim);
         TCHK(hipGetLastError());
-        TCHK(hipMemcpy(counts.data(), cnt.p, k * 4, hipMemcpyDeviceToHost));
+        TCHK(hipMemcpy(counts.data(), cnt, k * 4, hipMemcpyDeviceToHost));
         if (std::find(counts.begin(), counts.end(), 0u) != counts.end()) {
-            TCHK(hipMemcpy(init.data(), c.p, k * dim * 4, hipMemcpyDeviceToHost));
+            TCHK(hipMemcpy(init.data(), c, k * dim * 4, hipMemcpyDeviceToHost));
             if (split_empty_clusters(init, counts, (uint32_t)dim, split_gen))
-                TCHK(hipMemcpy(c.p, init.data(), k * dim * 4, hipMemcpyHostToDevice));
+                TCHK(hipMemcpy(c, init.data(), k * dim * 4, hipMemcpyHostToDevice));
         }
     }
     TCHK(hipDeviceSynchronize());
-    TCHK(hipMemcpy(h_centroids, c.p, k * dim * 4, hipMemcpyDeviceToHost));
+    TCHK(hipMemcpy(h_centroids, c, k * dim * 4, hipMemcpyDeviceToHost));
     return CORA_OK;
 }
 
@@ -664,44 +711,53 @@ int cora_tool_assign(const float *h_x, uint64_t n, uint64_t dim, const float *h_
     const size_t rows_dev = std::min<size_t>(n, 1u << 22);
     const size_t chunk = std::max<size_t>(1, std::min<size_t>(rows_dev, (size_t)(1u << 30) / (k * 4)));
     bool split = Nearest::supported(dim, k);
-    DevBuf x, c, cn, xn, dist, asg;
+    DevBlock block, split_block, fp32_block;
+    float *x, *c, *cn, *xn, *dist;
+    uint32_t *asg;
     Nearest near;
     SplitRows xs;
-    if (dev<float>(x, rows_dev * dim) || dev<float>(c, k * dim) || dev<uint32_t>(asg, rows_dev))
-        return CORA_ERR_RUNTIME;
+    block.add(x, rows_dev * dim);
+    block.add(c, k * dim);
+    block.add(asg, rows_dev);
+    TCHK(block.alloc());
     const size_t copy_rows = std::min(rows_dev, copy_chunk_rows(dim));
-    if (split && !(split = split_or_fp32(!near.init(dim, k, copy_rows) && !xs.alloc(copy_rows, near.Kp)))) {
-        near.release();
-        xs.release();
+    if (split) {
+        near.init(split_block, dim, k, copy_rows);
+        xs.add_to(split_block, copy_rows, near.Kp);
+        split = split_or_fp32(split_block);
     }
-    if (!split && (dev<float>(cn, k) || dev<float>(xn, chunk) || dev<float>(dist, chunk * k)))
-        return CORA_ERR_RUNTIME;
-    TCHK(hipMemcpy(c.p, h_centroids, k * dim * 4, hipMemcpyHostToDevice));
+    if (!split) {
+        fp32_block.add(cn, k);
+        fp32_block.add(xn, chunk);
+        fp32_block.add(dist, chunk * k);
+        TCHK(fp32_block.alloc());
+    }
+    TCHK(hipMemcpy(c, h_centroids, k * dim * 4, hipMemcpyHostToDevice));
     if (split) {
         if (int rc = near.set_shift(h_centroids))
             return rc;
-        near.set_centroids((float *)c.p, nullptr);
+        near.set_centroids(c, nullptr);
     } else
-        launch_row_norms((float *)c.p, (uint32_t)k, (uint32_t)dim, (float *)cn.p, nullptr);
+        launch_row_norms(c, (uint32_t)k, (uint32_t)dim, cn, nullptr);
     Staging st(device);
     for (size_t b = 0; b < n; b += rows_dev) {
         const size_t rows = std::min(rows_dev, n - b);
         int rc = 0;
-        TCHK(st.upload(h_x + b * dim, x.p, rows * dim * 4, copy_rows * dim * 4, rc, [&](size_t off, size_t len) {
+        TCHK(st.upload(h_x + b * dim, x, rows * dim * 4, copy_rows * dim * 4, rc, [&](size_t off, size_t len) {
             const size_t r0 = off / (dim * 4), m = len / (dim * 4);
-            float *xc = (float *)x.p + r0 * dim;
-            uint32_t *ac = (uint32_t *)asg.p + r0;
+            float *xc = x + r0 * dim;
+            uint32_t *ac = asg + r0;
             if (!split)
-                return assign_rows(xc, m, (uint32_t)dim, (float *)c.p, (float *)cn.p, (uint32_t)k, ac, (float *)xn.p,
-                                   (float *)dist.p, chunk, nullptr);
+                return assign_rows(xc, m, (uint32_t)dim, c, cn, (uint32_t)k, ac, xn,
+                                   dist, chunk, nullptr);
             xs.fill(xc, 0, (uint32_t)m, (uint32_t)dim, near.Kp, nullptr, near.shift);
-            near.assign(xc, xs, 0, m, (float *)c.p, ac, nullptr);
+            near.assign(xc, xs, 0, m, c, ac, nullptr);
             return (int)CORA_OK;
         }));
         if (rc)
             return rc;
         TCHK(hipGetLastError());
-        TCHK(hipMemcpy(h_assign + b, asg.p, rows * 4, hipMemcpyDeviceToHost));
+        TCHK(hipMemcpy(h_assign + b, asg, rows * 4, hipMemcpyDeviceToHost));
     }
     return CORA_OK;
 }
@@ -766,58 +822,68 @@ int topk_call(const float *h_base, uint64_t nb, const float *h_q, uint64_t nq, u
     const uint32_t Kp = split_padded(dim);
     bool split = blk * Kp < (1ull << 31) && qchunk * Kp < (1ull << 31);
     SplitRows bs, qs;
-    DevBuf b, bn, q, qn, dist, ids, cd, ci, out;
-    if (dev<float>(b, nb * dim) || dev<float>(bn, nb) || dev<float>(q, qchunk * dim) ||
-        dev<float>(qn, qchunk) || dev<float>(dist, qchunk * blk) || dev<int32_t>(ids, qchunk * k) ||
-        dev<float>(cd, qchunk * stride) || dev<uint32_t>(ci, qchunk * stride) || dev<uint32_t>(out, qchunk * k))
-        return CORA_ERR_RUNTIME;
-    if (split && !(split = split_or_fp32(!bs.alloc(nb, Kp) && !qs.alloc(qchunk, Kp)))) {
-        bs.release();
-        qs.release();
+    DevBlock block, split_block;
+    float *b, *bn, *q, *qn, *dist, *cd;
+    int32_t *ids;
+    uint32_t *ci, *out;
+    block.add(b, nb * dim);
+    block.add(bn, nb);
+    block.add(q, qchunk * dim);
+    block.add(qn, qchunk);
+    block.add(dist, qchunk * blk);
+    block.add(ids, qchunk * k);
+    block.add(cd, qchunk * stride);
+    block.add(ci, qchunk * stride);
+    block.add(out, qchunk * k);
+    TCHK(block.alloc());
+    if (split) {
+        bs.add_to(split_block, nb, Kp);
+        qs.add_to(split_block, qchunk, Kp);
+        split = split_or_fp32(split_block);
     }
     if (metric != 0) {  // an[m] + bn[n] - 2 * ip with zero norms = -2 ip: same order as -ip
-        TCHK(hipMemset(bn.p, 0, nb * 4));
-        TCHK(hipMemset(qn.p, 0, qchunk * 4));
+        TCHK(hipMemset(bn, 0, nb * 4));
+        TCHK(hipMemset(qn, 0, qchunk * 4));
     }
     const auto load_queries = [&](size_t s, size_t rows) -> int {
-        TCHK(hipMemcpy(q.p, h_q + s * dim, rows * dim * 4, hipMemcpyHostToDevice));
+        TCHK(hipMemcpy(q, h_q + s * dim, rows * dim * 4, hipMemcpyHostToDevice));
         if (split)
-            qs.fill((float *)q.p, 0, (uint32_t)rows, (uint32_t)dim, Kp, nullptr);
+            qs.fill(q, 0, (uint32_t)rows, (uint32_t)dim, Kp, nullptr);
         else if (metric == 0)
-            launch_row_norms((float *)q.p, (uint32_t)rows, (uint32_t)dim, (float *)qn.p, nullptr);
+            launch_row_norms(q, (uint32_t)rows, (uint32_t)dim, qn, nullptr);
         return CORA_OK;
     };
     // the k best of block j for the loaded queries
-    const auto block = [&](size_t j, size_t rows) {
+    const auto scan = [&](size_t j, size_t rows) {
         const size_t b0 = j * blk, len = std::min(blk, (size_t)nb - b0);
         if (split)
-            launch_dist_gemm_f16x3_rows((uint16_t *)qs.hi.p, (uint16_t *)qs.lo.p, (float *)qs.scale.p,
-                                        metric == 0 ? (float *)qs.norm.p : (float *)qn.p,
-                                        (uint16_t *)bs.hi.p + b0 * Kp, (uint16_t *)bs.lo.p + b0 * Kp,
-                                        (float *)bs.scale.p + b0,
-                                        (metric == 0 ? (float *)bs.norm.p : (float *)bn.p) + b0, (uint32_t)rows,
-                                        (uint32_t)len, Kp, (float *)dist.p, nullptr);
+            launch_dist_gemm_f16x3_rows(qs.hi, qs.lo, qs.scale,
+                                        metric == 0 ? qs.norm : qn,
+                                        bs.hi + b0 * Kp, bs.lo + b0 * Kp,
+                                        bs.scale + b0,
+                                        (metric == 0 ? bs.norm : bn) + b0, (uint32_t)rows,
+                                        (uint32_t)len, Kp, dist, nullptr);
         else
-            launch_dist_gemm((float *)q.p, (float *)qn.p, (float *)b.p + b0 * dim, (float *)bn.p + b0,
-                             (uint32_t)rows, (uint32_t)len, (uint32_t)dim, (float *)dist.p, nullptr);
-        launch_select((float *)dist.p, (uint32_t)rows, (uint32_t)len, (uint32_t)k, (int32_t *)ids.p, nullptr);
+            launch_dist_gemm(q, qn, b + b0 * dim, bn + b0,
+                             (uint32_t)rows, (uint32_t)len, (uint32_t)dim, dist, nullptr);
+        launch_select(dist, (uint32_t)rows, (uint32_t)len, (uint32_t)k, ids, nullptr);
         const size_t n = rows * k;
         gather_block_topk_kernel<<<(unsigned)((n + 255) / 256), 256>>>(
-            (float *)dist.p, (uint32_t)len, (int32_t *)ids.p, (uint32_t)rows, (uint32_t)k, (uint32_t)b0,
-            (uint32_t)stride, (uint32_t)(j * k), (float *)cd.p, (uint32_t *)ci.p);
+            dist, (uint32_t)len, ids, (uint32_t)rows, (uint32_t)k, (uint32_t)b0,
+            (uint32_t)stride, (uint32_t)(j * k), cd, ci);
     };
     Staging st(device);
     const size_t first = std::min<size_t>(qchunk, nq);
     if (int rc = load_queries(0, first))
         return rc;
     int rc = 0;
-    TCHK(st.upload(h_base, b.p, nb * dim * 4, blk * dim * 4, rc, [&](size_t off, size_t len) {
+    TCHK(st.upload(h_base, b, nb * dim * 4, blk * dim * 4, rc, [&](size_t off, size_t len) {
         const size_t r0 = off / (dim * 4), m = len / (dim * 4);
         if (split)
-            bs.fill((float *)b.p + r0 * dim, r0, (uint32_t)m, (uint32_t)dim, Kp, nullptr);
+            bs.fill(b + r0 * dim, r0, (uint32_t)m, (uint32_t)dim, Kp, nullptr);
         else if (metric == 0)
-            launch_row_norms((float *)b.p + r0 * dim, (uint32_t)m, (uint32_t)dim, (float *)bn.p + r0, nullptr);
-        block(r0 / blk, first);
+            launch_row_norms(b + r0 * dim, (uint32_t)m, (uint32_t)dim, bn + r0, nullptr);
+        scan(r0 / blk, first);
         return 0;
     }));
     for (size_t s = 0; s < nq; s += qchunk) {
@@ -826,17 +892,17 @@ int topk_call(const float *h_base, uint64_t nb, const float *h_q, uint64_t nq, u
             if ((rc = load_queries(s, rows)))
                 return rc;
             for (size_t j = 0; j < nblk; ++j)
-                block(j, rows);
+                scan(j, rows);
         }
         const size_t n = rows * k;
         if (nblk > 1)
-            launch_select((float *)cd.p, (uint32_t)rows, (uint32_t)stride, (uint32_t)k, (int32_t *)ids.p, nullptr);
+            launch_select(cd, (uint32_t)rows, (uint32_t)stride, (uint32_t)k, ids, nullptr);
         if (nblk > 1)
-            gather_ids_kernel<<<(unsigned)((n + 255) / 256), 256>>>((uint32_t *)ci.p, (uint32_t)stride,
-                                                                    (int32_t *)ids.p, (uint32_t)rows, (uint32_t)k,
-                                                                    (uint32_t *)out.p);
+            gather_ids_kernel<<<(unsigned)((n + 255) / 256), 256>>>(ci, (uint32_t)stride,
+                                                                    ids, (uint32_t)rows, (uint32_t)k,
+                                                                    out);
         TCHK(hipGetLastError());
-        TCHK(hipMemcpy(h_ids + s * k, nblk > 1 ? out.p : ci.p, n * 4, hipMemcpyDeviceToHost));
+        TCHK(hipMemcpy(h_ids + s * k, nblk > 1 ? out : ci, n * 4, hipMemcpyDeviceToHost));
     }
     return CORA_OK;
 }

@@ -341,16 +341,21 @@ int cora_gpu_debug_dense(cora_gpu_engine *engine, int32_t *out_ip, int32_t *out_
  * exhaustive ground-truth tool, tools/data/generate_gt_gpu.py). Host arrays in and out;
  * each call allocates and frees its own device memory on `device`. ---- */
 const char *cora_tool_last_error(void);
+/* For tests: while on, the calling thread's tools run as where their split-FP16 operands do not
+ * fit the device (the FP32 GEMM). Returns the previous setting. */
+int cora_tool_debug_no_split(int on);
 /* out [n][P] = x [n][dim] . R [dim][P] */
 int cora_tool_rotate(const float *x, uint64_t n, uint64_t dim, const float *R, uint64_t P,
                      float *out, int device);
 /* Lloyd k-means (squared L2), `iters` iterations from k seeded distinct rows. */
 int cora_tool_kmeans(const float *x, uint64_t n, uint64_t dim, uint64_t k, uint32_t iters,
                      uint64_t seed, float *centroids, int device);
-/* nearest centroid of every row (ties -> lower centroid id) */
+/* nearest centroid of every row in FP64 (ties -> lower centroid id); where the rows whose nearest
+ * centroids lie within the rounding of FP32 distances are many, the smallest such distance */
 int cora_tool_assign(const float *x, uint64_t n, uint64_t dim, const float *centroids, uint64_t k,
                      uint32_t *assign, int device);
-/* exhaustive top-k ids by FP32 distance (metric 0: L2, 1: IP), ascending */
+/* exhaustive top-k ids (metric 0: L2, 1: IP), ascending by distances to FP32 accuracy (split-FP16
+ * products, or FP32 ones where those operands do not fit) */
 int cora_tool_topk(const float *base, uint64_t nb, const float *queries, uint64_t nq, uint64_t dim,
                    uint64_t k, int metric, uint32_t *ids, int device);
 /* RaBitQ quantisation of index rows on the GPU (the index builder's per-row step,

@@ -425,3 +425,37 @@ def test_settling_many_rows_is_bounded(kind):
     t = call_seconds(lambda: ca.gpu_assign(x, c), 5)
     say(f"[tools] assign {n} x {dim}, k {k}: centred {centred * 1e3:.2f} ms, {kind} {t * 1e3:.2f} ms")
     assert t <= 3 * centred
+
+
+def test_fp32_path_where_the_split_operands_do_not_fit():
+    """What the tools do where the device has no room for the split-FP16 operands: assign still
+    gives the FP64 nearest (near ties and repeated centroids among the rows), k-means the means
+    of the rows nearest to its first ones, top-k the neighbours to FP32 accuracy."""
+    rng = np.random.default_rng(41)
+    n, dim, k = 9001, 100, 333
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    c = rng.standard_normal((k, dim)).astype(np.float32)
+    c[200] = c[7]
+    x[:100] = c[7] + 0.01 * x[:100]
+    x[100:200] = (c[5] + c[9]) / 2
+    q = rng.standard_normal((50, dim)).astype(np.float32)
+    say("[tools] the FP32 path")
+    gpu = ca.libs()[0]
+    was = gpu.cora_tool_debug_no_split(1)
+    try:
+        a = ca.gpu_assign(x, c).astype(np.int64)
+        first, mean = ca.gpu_kmeans(x, 40, 0, seed=1), ca.gpu_kmeans(x, 40, 1, seed=1)
+        tops = [ca.gpu_topk(x, q, 20, m) for m in (0, 1)]
+    finally:
+        gpu.cora_tool_debug_no_split(was)
+    d = np.stack([((r.astype(np.float64) - c.astype(np.float64)) ** 2).sum(1) for r in x])
+    got, best = d[np.arange(n), a], d.min(1)
+    assert np.all(got <= best * (1 + dim * 2.0 ** -50))
+    assert not np.any(a == 200)
+    near = fp64_nearest(x, first)[0]
+    for j in range(40):
+        rows = x[near == j].astype(np.float64)
+        tol = 2.0 ** -24 * (len(rows) + 2) * np.abs(rows).mean(0).max()
+        assert np.abs(mean[j] - rows.mean(0)).max() <= tol, j
+    for m in (0, 1):
+        check_topk(x, q, 20, m, tops[m])
