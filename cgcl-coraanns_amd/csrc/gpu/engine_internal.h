@@ -326,10 +326,11 @@ void launch_split_f16_rows(const float *x, uint32_t rows, uint32_t P, uint16_t *
 // the same from rows of P values to rows of Pp >= P (zeros between); norm (or nullptr): the rows'
 // squared norms
 // (copy: the rows themselves too, unless nullptr; shift [P]: subtracted from every row first, unless
-// nullptr)
+// nullptr; zeros [rows][P] and zero_counts [rows]: cleared in passing, unless nullptr)
 void launch_split_f16_padded(const float *x, uint32_t rows, uint32_t P, uint32_t Pp, uint16_t *hi, uint16_t *lo,
                              float *scale, float *norm, hipStream_t s, float *copy = nullptr,
-                             const float *shift = nullptr);
+                             const float *shift = nullptr, float *zeros = nullptr,
+                             uint32_t *zero_counts = nullptr);
 // an inner dimension rounded up to the split-FP16 GEMM's step
 uint32_t split_padded(uint64_t dim);
 // inner dimension K % 32 == 0 and rows * K < 2^31 for both operands
@@ -352,7 +353,7 @@ uint32_t nearest_tiles(uint32_t nl);
 void launch_nearest_gemm(const uint16_t *xhi, const uint16_t *xlo, const float *xscale, const float *xnorm,
                          const uint16_t *chi, const uint16_t *clo, const float *cscale, const float *cnorm,
                          uint32_t rows, uint32_t nl, uint32_t K, unsigned long long *best, uint32_t *second,
-                         hipStream_t s);
+                         uint32_t *counts /*[2], zeroed*/, hipStream_t s);
 // Fused coarse-probe select (fused_probe_supported: nl >= 8,192, nl <= kFusedProbeMaxList, and
 // nprobe <= 64, or up to 1,024 while a 128-cluster tile holds at most ~4.5 probes on average):
 // the split-FP16 distance GEMM keeps fused_probe_slots(nprobe) (8 or 16) candidate keys per

@@ -32,10 +32,11 @@ namespace cora {
 constexpr size_t kPieceBytes = size_t{4} << 20;
 constexpr int kCopyThreads = 4;  // 3, 4 and 6 copy alike
 constexpr int kKeepSets = 2;
-// Below these the runtime's copy is as fast. Up: plain 0.24 / 0.46 / 0.94 / 2.58 ms for 8, 16, 32
-// and 64 MiB, staged 0.27 / 0.46 / 0.82 / 1.58. Down: plain 0.25 / 0.49 / 0.98 / 2.03 for 4, 8, 16
-// and 32 MiB, staged 0.30 / 0.38 / 0.58 / 0.99.
-constexpr size_t kStagedUpBytes = size_t{32} << 20;
+// Below these the runtime's copy is as fast. Up: plain 0.24 / 0.46 / 0.94 / 1.43 / 2.58 ms for 8, 16,
+// 32, 40 and 64 MiB, staged 0.27 / 0.46 / 0.82 / 1.01 / 1.58 (a whole assign of 32 MiB: 1.25 and
+// 1.40 ms, of 64 MiB 2.77 and 2.41). Down: plain 0.25 / 0.49 / 0.98 / 2.03 for 4, 8, 16 and 32 MiB,
+// staged 0.30 / 0.38 / 0.58 / 0.99.
+constexpr size_t kStagedUpBytes = size_t{40} << 20;
 constexpr size_t kStagedDownBytes = size_t{8} << 20;
 
 struct StagingSet {

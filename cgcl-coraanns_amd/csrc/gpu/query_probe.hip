@@ -276,12 +276,13 @@ __device__ __forceinline__ int split_exponent(float amax) {
 
 // rows of P values (less shift [P], unless nullptr) to rows of Pp (zeros past P); copy: the values
 // too (nullptr: not wanted); norm: the rows' squared norms too, summed as row_norms_kernel sums
-// them (nullptr: not wanted)
+// them (nullptr: not wanted); zeros [rows][P], zero_counts [rows]: cleared (nullptr: none)
 __global__ __launch_bounds__(64) void split_f16_kernel(const float *__restrict__ x, uint32_t rows,
                                                        uint32_t P, uint32_t Pp, _Float16 *__restrict__ hi,
                                                        _Float16 *__restrict__ lo,
                                                        float *__restrict__ scale, float *__restrict__ norm,
-                                                       float *__restrict__ copy, const float *__restrict__ shift) {
+                                                       float *__restrict__ copy, const float *__restrict__ shift,
+                                                       float *__restrict__ zeros, uint32_t *__restrict__ zero_counts) {
     const int lane = threadIdx.x;
     for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x) {
         const float *row = x + (size_t)r * P;
@@ -304,6 +305,12 @@ __global__ __launch_bounds__(64) void split_f16_kernel(const float *__restrict__
         }
         if (lane == 0)
             scale[r] = ldexpf(1.0f, -e);
+        if (zeros) {
+            for (uint32_t i = lane; i < P; i += 64)
+                zeros[(size_t)r * P + i] = 0.0f;
+            if (lane == 0)
+                zero_counts[r] = 0;
+        }
         if (norm) {
             sq = wave_sum(sq);
             if (lane == 0)
@@ -367,7 +374,8 @@ constexpr int kEs = kHT + 4;  // LDS row stride (floats) of the epilogue's half 
 // written). kMode 3: distance rows of selected operand rows: output row m is A's row rmap[m],
 // for m < *mcount (at most M), the grid's row tiles sweeping them mstep rows at a time. kMode 4:
 // per row and 128-column tile the smallest (order key << 32 | column) to cand [M][ntiles] and the
-// order key of the second smallest distance to second [M][ntiles] (passed as C).
+// order key of the second smallest distance to second [M][ntiles] (passed as C); counts [2], which
+// the following kernel fills, are zeroed.
 // A [M][K] and B [N][K] are split-FP16 rows (Ah/Al, scale as; Bh/Bl, scale bs);
 // K % 32 == 0, rows 16-byte aligned. 128 x 128
 // output tile per workgroup of four waves (64 x 64 each, 4 x 4 MFMA blocks of 16 x 16),
@@ -383,12 +391,15 @@ __global__ __launch_bounds__(256, 3) void dist_gemm_f16x3_kernel(
     const _Float16 *__restrict__ Bh, const _Float16 *__restrict__ Bl, const float *__restrict__ bs,
     float *__restrict__ C, uint32_t M, uint32_t N, uint32_t K, const float *__restrict__ an,
     const float *__restrict__ bn, uint32_t ncx, uint32_t mstep, const uint32_t *__restrict__ rmap,
-    const uint32_t *__restrict__ mcount, unsigned long long *__restrict__ cand, uint32_t ntiles) {
+    const uint32_t *__restrict__ mcount, unsigned long long *__restrict__ cand, uint32_t ntiles,
+    uint32_t *__restrict__ counts = nullptr) {
     constexpr size_t kOperandBytes = 4 * kHT * 4 * sizeof(half8_t);
     constexpr size_t kHalfBytes = 64 * kEs * sizeof(float);
     constexpr size_t kLdsBytes = kMode == 2 && kHalfBytes > kOperandBytes ? kHalfBytes : kOperandBytes;
     __shared__ __align__(16) unsigned char s_raw[kLdsBytes];
     half8_t(*S)[kHT * 4] = reinterpret_cast<half8_t(*)[kHT * 4]>(s_raw);  // [Ah, Al, Bh, Bl][row x group]
+    if (kMode == 4 && blockIdx.x == 0 && threadIdx.x < 2)
+        counts[threadIdx.x] = 0;
     uint32_t rt, ct;
     tile_of(blockIdx.x, ncx, (N + kHT - 1) / kHT, rt, ct);
     const uint32_t n0 = ct * kHT;
@@ -1864,12 +1875,13 @@ void launch_split_f16_rows(const float *x, uint32_t rows, uint32_t P, uint16_t *
 uint32_t split_padded(uint64_t dim) { return (uint32_t)((dim + kHK - 1) / kHK * kHK); }
 
 void launch_split_f16_padded(const float *x, uint32_t rows, uint32_t P, uint32_t Pp, uint16_t *hi, uint16_t *lo,
-                             float *scale, float *norm, hipStream_t s, float *copy, const float *shift) {
+                             float *scale, float *norm, hipStream_t s, float *copy, const float *shift, float *zeros,
+                             uint32_t *zero_counts) {
     if (!rows)
         return;
     split_f16_kernel<<<rows < (1u << 20) ? rows : (1u << 20), 64, 0, s>>>(
         x, rows, P, Pp, reinterpret_cast<_Float16 *>(hi), reinterpret_cast<_Float16 *>(lo), scale, norm, copy,
-        shift);
+        shift, zeros, zero_counts);
 }
 
 bool dist_gemm_f16x3_supported(uint32_t K, uint64_t rows_a, uint64_t rows_b) {
@@ -1903,7 +1915,7 @@ uint32_t nearest_tiles(uint32_t nl) { return (nl + kHT - 1) / kHT; }
 void launch_nearest_gemm(const uint16_t *xhi, const uint16_t *xlo, const float *xscale, const float *xnorm,
                          const uint16_t *chi, const uint16_t *clo, const float *cscale, const float *cnorm,
                          uint32_t rows, uint32_t nl, uint32_t K, unsigned long long *best, uint32_t *second,
-                         hipStream_t s) {
+                         uint32_t *counts, hipStream_t s) {
     if (!rows || !nl)
         return;
     const uint32_t nct = nearest_tiles(nl);
@@ -1911,7 +1923,8 @@ void launch_nearest_gemm(const uint16_t *xhi, const uint16_t *xlo, const float *
     dist_gemm_f16x3_kernel<4><<<o.blocks, 256, 0, s>>>(
         reinterpret_cast<const _Float16 *>(xhi), reinterpret_cast<const _Float16 *>(xlo), xscale,
         reinterpret_cast<const _Float16 *>(chi), reinterpret_cast<const _Float16 *>(clo), cscale,
-        reinterpret_cast<float *>(second), rows, nl, K, xnorm, cnorm, o.cols, 0, nullptr, nullptr, best, nct);
+        reinterpret_cast<float *>(second), rows, nl, K, xnorm, cnorm, o.cols, 0, nullptr, nullptr, best, nct,
+        counts);
 }
 
 bool fused_probe_supported(uint32_t nl, uint32_t nprobe) {

@@ -388,9 +388,9 @@ struct SplitRows {
         block.add(norm, rows);
     }
     void fill(const float *d_x, size_t row0, uint32_t rows, uint32_t dim, uint32_t Kp, hipStream_t s,
-              const float *shift = nullptr) {
+              const float *shift = nullptr, float *zeros = nullptr, uint32_t *zero_counts = nullptr) {
         launch_split_f16_padded(d_x, rows, dim, Kp, hi + row0 * Kp, lo + row0 * Kp, scale + row0, norm + row0, s,
-                                nullptr, shift);
+                                nullptr, shift, zeros, zero_counts);
     }
 };
 
@@ -421,30 +421,34 @@ struct Nearest {
         block.add(count, 2);
         block.add(offset, dim);
     }
-    // The mean of up to 256 of the (host) centroids, where it is longer than their spread about it:
+    // The mean of up to 64 of the (host) centroids, where it is longer than their spread about it:
     // taking away less would not make the norms much smaller.
     int set_shift(const float *h_c) {
-        const size_t step = std::max<size_t>(1, k / 256), n = (k + step - 1) / step;
-        std::vector<double> sum(dim, 0.0);
-        double square = 0.0, offset2 = 0.0;
+        const size_t step = std::max<size_t>(1, k / 64), n = (k + step - 1) / step;
+        std::vector<double> sum(dim, 0.0), squares(dim, 0.0);
         for (size_t i = 0; i < k; i += step)
             for (uint32_t d = 0; d < dim; ++d) {
                 const double v = h_c[i * dim + d];
                 sum[d] += v;
-                square += v * v;
+                squares[d] += v * v;
             }
         std::vector<float> mean(dim);
+        double square = 0.0, offset2 = 0.0;
         for (uint32_t d = 0; d < dim; ++d) {
             mean[d] = (float)(sum[d] / (double)n);
             offset2 += (double)mean[d] * mean[d];
+            square += squares[d] / (double)n;
         }
-        if (!(offset2 > 0.5 * square / (double)n && offset2 < (double)FLT_MAX))  // nor where it is not finite
+        if (!(offset2 > 0.5 * square && offset2 < (double)FLT_MAX))  // nor where it is not finite
             return CORA_OK;
         TCHK(hipMemcpy(offset, mean.data(), dim * 4, hipMemcpyHostToDevice));
         shift = offset;
         return CORA_OK;
     }
-    void set_centroids(const float *d_c, hipStream_t s) { c.fill(d_c, 0, k, dim, Kp, s, shift); }
+    // (k-means: its sums [k][dim] and counts [k] cleared)
+    void set_centroids(const float *d_c, hipStream_t s, float *sums = nullptr, uint32_t *counts = nullptr) {
+        c.fill(d_c, 0, k, dim, Kp, s, shift, sums, counts);
+    }
     // rows [r0, r0 + n) of x (split in xs from row s0): assign[r0 ..]
     void assign(const float *d_x, const SplitRows &xs, size_t s0, size_t n, const float *d_c, uint32_t *d_assign,
                 hipStream_t s) {
@@ -452,12 +456,11 @@ struct Nearest {
             const uint32_t rows = (uint32_t)std::min(chunk, n - b);
             const size_t at = s0 + b;
             const float *xn = xs.norm + at;
-            launch_fill_u32(count, 0u, 2, s);
             launch_nearest_gemm(xs.hi + at * Kp, xs.lo + at * Kp, xs.scale + at, xn, c.hi, c.lo, c.scale, c.norm, rows,
-                                k, Kp, best, second, s);
+                                k, Kp, best, second, count, s);
             nearest_rows_kernel<<<(rows + 3) / 4, 256, 0, s>>>(best, second, rows, tiles, xn, dim, d_assign + b, list,
                                                                count);
-            nearest_exact_kernel<<<std::min<uint32_t>(rows, 2048), 256, 0, s>>>(best, second, tiles, d_x + b * dim, xn,
+            nearest_exact_kernel<<<std::clamp<uint32_t>(rows / 8, 256, 2048), 256, 0, s>>>(best, second, tiles, d_x + b * dim, xn,
                                                                                 d_c, k, dim, list, count, rows,
                                                                                 d_assign + b);
         }
@@ -674,17 +677,15 @@ int cora_tool_kmeans(const float *h_x, uint64_t n, uint64_t dim, uint64_t k, uin
     std::mt19937_64 split_gen(seed ^ 0x9E3779B97F4A7C15ull);
     for (uint32_t it = 0; it < iters; ++it) {
         if (split) {
-            near.set_centroids(c, nullptr);
+            near.set_centroids(c, nullptr, sums, cnt);
             near.assign(x, xs, 0, n, c, asg, nullptr);
         } else {
             launch_row_norms(c, (uint32_t)k, (uint32_t)dim, cn, nullptr);
-            if (int rc = assign_rows(x, n, (uint32_t)dim, c, cn,
-                                     (uint32_t)k, asg, xn, dist,
-                                     chunk, nullptr))
+            if (int rc = assign_rows(x, n, (uint32_t)dim, c, cn, (uint32_t)k, asg, xn, dist, chunk, nullptr))
                 return rc;
+            TCHK(hipMemset(sums, 0, k * dim * 4));
+            TCHK(hipMemset(cnt, 0, k * 4));
         }
-        TCHK(hipMemset(sums, 0, k * dim * 4));
-        TCHK(hipMemset(cnt, 0, k * 4));
         accumulate_kernel<<<(uint32_t)std::min<uint64_t>(n, 1u << 20), 64>>>(x, asg, (uint32_t)n,
                                                 (uint32_t)dim, sums, cnt);
         update_kernel<<<(uint32_t)((k * dim + 255) / 256), 256>>>(c, sums,
