@@ -973,12 +973,13 @@ int cora_gpu_launch_search(cora_gpu_engine *E, const cora_search_args *a) {
     // padded dimension allows it (the unit size changes only the speed, never the result).
     // The LUT4 estimator (the reference's default Lut4Bit producers) runs the per-pair seed,
     // far and recovery passes of the popcount kernels with the FP16 tables in place of the
-    // q-planes, at most kLutMaxBatchQ pairs per pass.
+    // q-planes, at most kLutMaxBatchQ pairs per pass, where the matrix cores do not take over.
     const bool reuse = (a->flags & CORA_FLAG_CROSS_QUERY_REUSE) != 0;
-    // LUT4 on the matrix cores (wide codes): the far scan and the vanguard lows pass filter
-    // with Bitwise bounds lowered by the query's LUT4 margin and evaluate the LUT4 bound of
-    // the survivors exactly; the vanguard pass is the staged one, refining with the LUT4
-    // estimate
+    // LUT4 on the matrix cores (P >= 128): the far scan filters with Bitwise bounds lowered by the
+    // query's LUT4 margin and evaluates the LUT4 bound of the survivors exactly. From kLowsMinDim,
+    // where the staged vanguard pass is built (lut_staged below), so does the lows pass and that
+    // pass refines with the LUT4 estimate; elsewhere the vanguard pairs run in the per-pair
+    // passes.
     const bool lut_mfma = lut && reuse && far_mfma_lut_supported(E->W) && !(a->flags & CORA_FLAG_NO_MFMA_SCAN);
     const bool mfma_far = (!lut || lut_mfma) && reuse && far_mfma_supported(E->W) &&
                           !(a->flags & CORA_FLAG_NO_MFMA_SCAN);

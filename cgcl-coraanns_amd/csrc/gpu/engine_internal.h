@@ -289,7 +289,9 @@ struct VsArgs {
 };
 
 // the staged pass: P of 64..1024 with a compiled refinement kernel
-bool vanguard_staged_supported(uint32_t W);
+constexpr bool vanguard_staged_supported(uint32_t W) {
+    return W == 2 || W == 4 || W == 8 || W == 16 || W == 24 || W == 32;
+}
 // refine_ms: optional events around the two refinement launches (timing)
 void launch_vanguard_staged(const ScanParams &p, const VanguardArgs &va, const VsArgs &vs, uint32_t W, uint32_t nq,
                             hipEvent_t ev_r0, hipEvent_t ev_r1, hipEvent_t ev_r2, hipEvent_t ev_r3, hipStream_t s);
@@ -448,7 +450,7 @@ constexpr uint32_t kLutMaxBatchQ = 4;
 // far-pair scan on the matrix cores (scan_mfma.hip): units of up to kMfmaBatchQ pairs
 constexpr uint32_t kMfmaBatchQ = 16;
 bool far_mfma_supported(uint32_t W);
-// the LUT4 estimator on the matrix-core kernels (P = 128, 256, 384, 512, 768, 1024)
+// the LUT4 estimator in the matrix-core far scan (P = 128 .. 1024)
 bool far_mfma_lut_supported(uint32_t W);
 void launch_far_mfma(const ScanParams &p, uint32_t W, bool dense, hipStream_t s);
 // The vanguard units (units of up to kMfmaBatchQ pairs, set 0) on the matrix cores: the lower

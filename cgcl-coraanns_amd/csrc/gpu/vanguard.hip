@@ -1057,9 +1057,14 @@ void launch_vanguard_query(const ScanParams &p, const VanguardArgs &va, uint32_t
     case 8: launch_vq_w<8>(p, va, nq, s); break;
     case 10: launch_vq_w<10>(p, va, nq, s); break;
     case 12: launch_vq_w<12>(p, va, nq, s); break;
+    case 14: launch_vq_w<14>(p, va, nq, s); break;
     case 16: launch_vq_w<16>(p, va, nq, s); break;
+    case 18: launch_vq_w<18>(p, va, nq, s); break;
     case 20: launch_vq_w<20>(p, va, nq, s); break;
+    case 22: launch_vq_w<22>(p, va, nq, s); break;
     case 24: launch_vq_w<24>(p, va, nq, s); break;
+    case 26: launch_vq_w<26>(p, va, nq, s); break;
+    case 28: launch_vq_w<28>(p, va, nq, s); break;
     case 30: launch_vq_w<30>(p, va, nq, s); break;
     case 32: launch_vq_w<32>(p, va, nq, s); break;
     default: launch_vq_w<0>(p, va, nq, s); break;

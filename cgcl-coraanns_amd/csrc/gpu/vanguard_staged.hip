@@ -1063,10 +1063,6 @@ void launch_vs_w(const ScanParams &p, const VanguardArgs &va, const VsArgs &vs, 
 
 }  // namespace
 
-bool vanguard_staged_supported(uint32_t W) {
-    return W == 2 || W == 4 || W == 8 || W == 16 || W == 24 || W == 32;
-}
-
 void launch_vanguard_staged(const ScanParams &p, const VanguardArgs &va, const VsArgs &vs, uint32_t W, uint32_t nq,
                             hipEvent_t ev_r0, hipEvent_t ev_r1, hipEvent_t ev_r2, hipEvent_t ev_r3, hipStream_t s) {
     if (nq == 0 || va.depth == 0)

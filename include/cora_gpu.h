@@ -99,10 +99,10 @@ enum cora_search_flags {
     /* LUT4 estimator, the reference's KernelType::Lut4Bit (query_kernels.cuh:199-221,
      * filter_kernels.cuh:283-306,586-770): <q',b> is the FP32 sum of FP16 nibble-table
      * entries (even and odd nibbles in two accumulators), used for the lower bound and handed
-     * to refinement as exact_ip. For padded dimension 128, 256, 384, 512, 768 or 1024 with
-     * cross-query reuse, the matrix-core far scan filters with Bitwise bounds lowered by a
-     * per-query bound on |LUT4 - Bitwise| and evaluates the survivors' LUT4 bounds exactly; from
-     * 512 the lows pass does too, and the staged vanguard pass refines with the LUT4 estimate.
+     * to refinement as exact_ip. For padded dimensions from 128 with cross-query reuse, the
+     * matrix-core far scan filters with Bitwise bounds lowered by a per-query bound on
+     * |LUT4 - Bitwise| and evaluates the survivors' LUT4 bounds exactly; at 512, 768 and 1024
+     * the lows pass does too, and the staged vanguard pass refines with the LUT4 estimate.
      * Otherwise the per-pair seed, far and recovery passes run with at most 4 same-cluster
      * pairs per pass.
      * Without it the Bitwise estimator runs (Bq=8 popcount bound; two-stage exact_ip). */

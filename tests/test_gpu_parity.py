@@ -1630,3 +1630,9 @@ def test_lut4_far_scan_on_the_matrix_cores(dim, tmp_path_factory):
                 eng.close()
         for o in out[1:]:
             assert np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1]) and o[2] == out[0][2]
+
+
+@pytest.mark.parametrize("dim", [192, 320, 576, 704, 832, 960])
+def test_lut4_far_scan_at_other_widths(dim, tmp_path_factory):
+    """The same at widths of odd lane-group shares, of padding words and of a two-word last group."""
+    test_lut4_far_scan_on_the_matrix_cores(dim, tmp_path_factory)
