@@ -149,7 +149,7 @@ struct cora_gpu_engine {
     unsigned long long *h_sync = nullptr;  // pinned: the search's statistics and stall flag (cora_gpu_sync)
     int *h_abort = nullptr;
     unsigned long long *d_produced = nullptr, *d_cached_limit = nullptr, *d_spill_count = nullptr;
-    int *d_refresh = nullptr, *d_overflow = nullptr, *d_stalled = nullptr;
+    int *d_refresh = nullptr, *d_overflow = nullptr;
     SpillRecord *d_spill = nullptr;
     bool ring_dirty = false;
     bool final_mode = false;  // the launch in flight publishes to HBM (CORA_FLAG_GPU_FINAL)
@@ -204,7 +204,6 @@ QueueDev queue_dev(cora_gpu_engine *E) {
     q.spill_capacity = E->spill_cap;
     q.spill_overflow = E->d_overflow;
     q.abort_flag = E->h_abort;
-    q.stalled = E->d_stalled;
     q.final_mode = E->final_mode ? 1 : 0;
     return q;
 }
@@ -266,7 +265,6 @@ void release_queue(cora_gpu_engine *E) {
     dfree(E->d_spill_count);
     dfree(E->d_refresh);
     dfree(E->d_overflow);
-    dfree(E->d_stalled);
     dfree(E->d_spill);
 }
 
@@ -791,7 +789,6 @@ int cora_gpu_prepare_workspace(cora_gpu_engine *E, uint64_t max_q, uint64_t max_
         TRY(dalloc(E, E->d_spill_count, 1));
         TRY(dalloc(E, E->d_refresh, 1));
         TRY(dalloc(E, E->d_overflow, 1));
-        TRY(dalloc(E, E->d_stalled, 1));
         TRY(dalloc(E, E->d_spill, std::max<uint64_t>(1, E->spill_cap)));
         return CORA_OK;
     };

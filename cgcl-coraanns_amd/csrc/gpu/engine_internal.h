@@ -137,7 +137,6 @@ struct QueueDev {
     unsigned long long spill_capacity;
     int *spill_overflow;
     int *abort_flag;                   // host-coherent
-    int *stalled;                      // HBM
     // GPU-final top-k: records go to spill[position].item (not to the ring) and carry the
     // refined distance in place of exact_ip
     int final_mode;

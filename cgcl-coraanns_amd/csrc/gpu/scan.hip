@@ -748,7 +748,6 @@ __global__ void queue_reset_kernel(QueueDev q) {
     *q.spill_overflow = 0;
     *q.cached_limit = q.capacity;
     *q.refresh_flag = 0;
-    *q.stalled = 0;
 }
 
 __global__ void cursor_init_kernel(uint32_t *cursor, const uint32_t *num_units, uint32_t set) {
@@ -834,8 +833,6 @@ __global__ __launch_bounds__(256) void finish_kernel(QueueDev q, unsigned long l
     if (t == 11)
         host_stats[11] = stalled ? 1ull : 0ull;
     if (t == 0) {
-        if (stalled)
-            *q.stalled = 1;
         __threadfence_system();
         if (overflow || stalled)
             __hip_atomic_store(&q.progress->overflow, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
