@@ -12,6 +12,7 @@
 #include <math.h>
 
 #include "engine_internal.h"
+#include "lane_ops.h"
 #include "tile_order.h"
 
 namespace cora {
@@ -343,21 +344,6 @@ __device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t x)
     return r;
 }
 
-// The value of lane ^ kMask within each row of 16 lanes (DPP moves: quad permutations, the half
-// mirror and the rotation by 8)
-template <int kMask>
-__device__ __forceinline__ uint32_t row_xor(uint32_t v) {
-    if constexpr (kMask == 1)
-        return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
-    else if constexpr (kMask == 2)
-        return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
-    else if constexpr (kMask == 4)  // 7 ^ 3: half mirror, then each quad reversed
-        return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true), 0x1B, 0xF,
-                                           0xF, true);
-    else
-        return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);
-}
-
 // Fused probe select: the GEMM epilogue keeps, per query row and 128-cluster tile, the
 // kSlots smallest (distance, cluster) keys (kProbeSlots, or kProbeSlotsWide for larger
 // nprobe), compared on the order key with its low 7 bits
@@ -505,10 +491,10 @@ __global__ __launch_bounds__(256, 3) void dist_gemm_f16x3_kernel(
                         k1 = take ? ok1 : k1;
                         c1 = take ? oc1 : c1;
                     };
-                    merge(row_xor<1>(k1), row_xor<1>(c1), row_xor<1>(k2));
-                    merge(row_xor<2>(k1), row_xor<2>(c1), row_xor<2>(k2));
-                    merge(row_xor<4>(k1), row_xor<4>(c1), row_xor<4>(k2));
-                    merge(row_xor<8>(k1), row_xor<8>(c1), row_xor<8>(k2));
+                    merge(lane_xor<1>(k1), lane_xor<1>(c1), lane_xor<1>(k2));
+                    merge(lane_xor<2>(k1), lane_xor<2>(c1), lane_xor<2>(k2));
+                    merge(lane_xor<4>(k1), lane_xor<4>(c1), lane_xor<4>(k2));
+                    merge(lane_xor<8>(k1), lane_xor<8>(c1), lane_xor<8>(k2));
                     if (i16 == 0) {
                         uint32_t *b = s_best[wave & 1][wm + 16 * ti + 4 * g + r];
                         b[0] = k1;
