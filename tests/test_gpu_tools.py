@@ -58,23 +58,28 @@ def test_topk_single_block(metric):
 
 @pytest.mark.parametrize("metric", [0, 1])
 def test_topk_two_level_blocks(metric):
-    """More than 2^20 base rows: blocks of the base selected separately and merged; the
-    true neighbours are planted in the last block, across the block boundary and in the
-    first block, so a merge that drops a block fails."""
+    """A base of several blocks, selected separately and merged: the true neighbours are planted
+    on both sides of every block boundary and at both ends, so a merge that drops a block or a
+    block's edge fails."""
     rng = np.random.default_rng(5 + metric)
     nb, dim, nq, k = (1 << 21) + 777, 16, 24, 26
     base = rng.standard_normal((nb, dim)).astype(np.float32)
     q = rng.standard_normal((nq, dim)).astype(np.float32)
-    blk = (nb + 2) // 3  # three blocks of the tool's split
-    for i in range(nq):
-        where = [nb - 1 - i, blk - 1 - i, blk + i, i][i % 4]
-        base[where] = q[i] * (1.5 if metric == 1 else 1.0)
+    # the tool's split: blocks of about 2^18 rows where their candidates number 4,096 at most
+    nblk = -(-nb >> 18)
+    assert nblk * k <= 4096
+    blk = -(-nb // nblk)
+    assert nblk == 9 and nb - (nblk - 1) * blk > nq  # the last block is a little shorter
+    where = [0, nb - 1] + [j * blk + e for j in range(1, nblk) for e in (-1, 0)]
+    where += [j * blk + 1 for j in range(1, 1 + nq - len(where))]
+    assert len(set(where)) == nq
+    for w, v in zip(where, q):
+        base[w] = v * (1.5 if metric == 1 else 1.0)
     say(f"[tools] topk two-level metric={metric} nb={nb}")
     ids = ca.gpu_topk(base, q, k, metric)
     check_topk(base, q, k, metric, ids)
     for i in range(nq):
-        where = [nb - 1 - i, blk - 1 - i, blk + i, i][i % 4]
-        assert where in ids[i]
+        assert where[i] in ids[i]
 
 
 def test_topk_k_equals_nb():
@@ -140,8 +145,8 @@ def test_kmeans_reseeds_empty_clusters():
 
 @pytest.mark.parametrize("dim,P,metric", [(128, 128, 0), (128, 128, 1), (250, 256, 0), (768, 768, 1)])
 def test_gpu_builder_matches_host_builder(dim, P, metric, tmp_path):
-    """The GPU quantiser (cora_build_ivf_gpu) writes the same index file, byte for byte, as
-    the host builder (cora_build_ivf, itself pinned to the reference builder's codes) on the
+    """The GPU quantiser (cora_build_ivf_gpu) writes the same index file, byte for byte (no row here
+    has its best t below the GPU sweep's start), as the host builder (cora_build_ivf, itself pinned to the reference builder's codes) on the
     GPU-rotated rows: sign codes, all factors, ex-codes, ids."""
     rng = np.random.default_rng(dim + metric)
     n, nl = 3000, 12
