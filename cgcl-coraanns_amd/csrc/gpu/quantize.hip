@@ -1,6 +1,8 @@
-// RaBitQ quantisation of index rows on the GPU (index build), bit-identical to the host
-// builder (csrc/host/index.cpp, which restates rabitq_impl.hpp:76-137 one_bit_code_with_factor,
-// 276-333 best_rescale_factor, 336-360 quantize_ex and 405-500 ex_bits_code_with_factor).
+// RaBitQ quantisation of index rows on the GPU (index build): the sign codes and their factors are
+// the host builder's bit for bit (csrc/host/index.cpp, which restates rabitq_impl.hpp:76-137
+// one_bit_code_with_factor, 276-333 best_rescale_factor, 336-360 quantize_ex and 405-500
+// ex_bits_code_with_factor), the ex-codes and theirs at every row whose best t lies at or above
+// kQzTight * t_end (see there).
 //
 // One wave per row. The host forms its double-precision sums in index order. Most of them
 // become floats: the sum is formed in parallel here and taken where every value within the
@@ -51,8 +53,10 @@ constexpr int kQzWin = 1024;          // events per sorted window
 constexpr int kQzTarget = 896;        // events per window aimed at
 constexpr int kQzCap = 127;           // 2^7 - 1 (7 ex-bits)
 constexpr int kQzNEnum = 10;
-// where the sweep starts, as a share of t_end (the host starts at 0.77, kTightStart[7] of
-// rabitq_impl.hpp:263-273: rows whose best t lies between differ)
+// Where the sweep starts, as a share of t_end. The host starts at 0.77 (kTightStart[7] of
+// rabitq_impl.hpp:263-273), so a row whose best t lies between gets the best code from 0.81 up
+// here: on Gaussian mixtures 1,630 of 300,000 rows at P = 64, about 55 of 200,000 at 128, 1 of
+// 100,000 at 256, none of 340,000 at 384 to 1,024.
 constexpr double kQzTight = 0.81;
 constexpr double kQzEps = 1e-5;
 constexpr float kQzConstEpsilon = 1.9f;  // rabitq_impl.hpp:18

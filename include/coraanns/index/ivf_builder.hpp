@@ -24,8 +24,9 @@ struct BuildInput {
 
 IvfFile build_ivf(const BuildInput &in, int threads = 0);
 
-// The same index from raw rows, rotated and quantised on GPU `device` (cora_tool_quantize,
-// bit-identical to build_ivf on the GPU-rotated rows); the host packs the codes.
+// The same index from raw rows, rotated and quantised on GPU `device` (cora_tool_quantize: build_ivf's
+// codes and factors on the GPU-rotated rows, but for the ex-codes of the few rows named there);
+// the host packs the codes.
 struct GpuBuildInput {
     const float *data = nullptr;               // [n][dim] raw rows
     const float *rotated_centroids = nullptr;  // [nlist][padded_dim]
