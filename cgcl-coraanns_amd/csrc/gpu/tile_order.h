@@ -25,11 +25,13 @@ struct TileOrder {
 };
 
 // The order whose busiest XCD has fewer tiles; by columns unless rows save an eighth of them (the
-// sweep by rows reads the column operand once per XCD and group).
+// sweep by rows reads the column operand once per XCD and group), and while the busiest has at
+// most 16 of them, for half its 32 CUs: nothing queues then (777 queries of 384 dimensions against
+// 1,500 centroids, 14 tiles by columns and 12 by rows: 24.7 and 30.3 us).
 inline TileOrder tile_order(uint32_t row_tiles, uint32_t col_tiles) {
     const uint32_t cols = (col_tiles + 7) / 8, rows = (row_tiles + 7) / 8;
     const uint64_t by_cols = (uint64_t)cols * row_tiles, by_rows = (uint64_t)rows * col_tiles;
-    if (8 * by_rows < 7 * by_cols)
+    if (by_cols > 16 && 8 * by_rows < 7 * by_cols)
         return {0, 8 * 4 * col_tiles * ((rows + 3) / 4)};
     return {cols, 8 * 4 * cols * ((row_tiles + 3) / 4)};
 }
