@@ -396,8 +396,8 @@ struct SplitRows {
 
 // Nearest centroids on the FP16 matrix cores (three FP16 products per term; FP32 has no fast
 // matrix path): the distance matrix is never written, 12 bytes per row and 128 centroids
-// are. 300,000 x 768 against 8,192: GEMM and argmin 39.4 -> 13.9 ms; k-means of
-// 262,144 x 128, k = 1,024: 1.35 -> 0.75 ms an iteration.
+// are. 300,000 x 768 against 8,192: GEMM and argmin 39.4 -> 12.1 ms; k-means of
+// 262,144 x 128, k = 1,024: 1.35 -> 0.66 ms an iteration.
 struct Nearest {
     uint32_t dim = 0, Kp = 0, k = 0, tiles = 0;
     size_t chunk = 0;
@@ -912,8 +912,9 @@ int topk_call(const float *h_base, uint64_t nb, const float *h_q, uint64_t nq, u
 
 extern "C" {
 
-// Exhaustive top-k of nq queries over nb base rows by FP32 distance (L2: ||q-x||^2 through
-// the norm expansion; IP: -<q,x>), ascending, ties by base index. Callers that need the
+// Exhaustive top-k of nq queries over nb base rows by distances to FP32 accuracy (L2: ||q-x||^2
+// through the norm expansion; IP: -<q,x>; split-FP16 products, no further from 64 bits than the
+// FP32 GEMM's where measured, dimensions 64 to 1,024), ascending, ties by base index. Callers that need the
 // exact order re-rank a few extra candidates in FP64.
 int cora_tool_topk(const float *h_base, uint64_t nb, const float *h_q, uint64_t nq, uint64_t dim,
                    uint64_t k, int metric, uint32_t *h_ids, int device) {
