@@ -1,7 +1,7 @@
 // Index-build and evaluation tools on the GPU (C-ABI in include/cora_gpu.h, cora_tool_*):
 // rotation of a row block, Lloyd k-means, nearest-centroid assignment and exhaustive
 // top-k (ground truth). They reuse the engine's split-FP16 and FP32 GEMMs, row-norm and top-k
-// select kernels; host arrays in, host arrays out, device memory allocated per call.
+// select kernels; host arrays in, host arrays out, device memory in a block a call (dev_block.h).
 #include <float.h>
 #include <stdio.h>
 #include <string.h>

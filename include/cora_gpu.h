@@ -339,7 +339,8 @@ int cora_gpu_debug_dense(cora_gpu_engine *engine, int32_t *out_ip, int32_t *out_
 /* ---- Index-build and evaluation tools (no counterpart in the reference's search path;
  * they replace its offline Faiss k-means, tools/data/train_ivf.py:11-47, and the
  * exhaustive ground-truth tool, tools/data/generate_gt_gpu.py). Host arrays in and out;
- * each call allocates and frees its own device memory on `device`. ---- */
+ * each call takes its own device memory on `device` (two blocks of up to 256 MiB are kept for
+ * later calls). ---- */
 const char *cora_tool_last_error(void);
 /* For tests: while on, the calling thread's tools run as where their split-FP16 operands do not
  * fit the device (the FP32 GEMM). Returns the previous setting. */

@@ -464,3 +464,22 @@ def test_fp32_path_where_the_split_operands_do_not_fit():
         assert np.abs(mean[j] - rows.mean(0)).max() <= tol, j
     for m in (0, 1):
         check_topk(x, q, 20, m, tops[m])
+
+
+def test_calls_of_changing_sizes():
+    """Calls take their device arrays from blocks that earlier calls of other sizes left: whatever
+    these hold, every call gives its own answer."""
+    rng = np.random.default_rng(51)
+    say("[tools] calls of changing sizes")
+    for n, dim, k in [(9000, 100, 40), (200, 33, 7), (30_000, 64, 300), (5, 3, 2), (700, 384, 129), (30_000, 31, 5)]:
+        c = rng.standard_normal((k, dim)).astype(np.float32)
+        x = (c[rng.integers(0, k, n)] + rng.standard_normal((n, dim))).astype(np.float32)
+        want, gap = fp64_nearest(x, c)
+        assert gap.min() > 1e-9
+        assert np.array_equal(ca.gpu_assign(x, c), want)
+        q = rng.standard_normal((9, dim)).astype(np.float32)
+        for metric in (0, 1):
+            check_topk(x, q, 5, metric, ca.gpu_topk(x, q, 5, metric))
+        R = np.linalg.qr(rng.standard_normal((dim, dim)))[0].astype(np.float32)
+        tol = dim * 2.0 ** -24 * np.linalg.norm(x, axis=1).max()
+        assert np.abs(ca.gpu_rotate(x, R) - x.astype(np.float64) @ R.astype(np.float64)).max() < tol
