@@ -378,7 +378,9 @@ int cora_tool_quantize(const float *x, uint64_t n, uint64_t dim, const float *R,
  * loops that assign new vectors to clusters, harnesses that forbid hipMalloc). x [n][dim],
  * centroids [k][dim] and assign [n] are DEVICE arrays on `device`, owned by the caller; the
  * norms and distance blocks go to a 16 MiB static device array that each GPU holds until the
- * process ends. Same result as cora_tool_assign (nearest centroid, ties -> lower id). At most
+ * process ends. Same result as cora_tool_assign (nearest centroid, ties -> lower id), but for
+ * rows with more than 16 centroids within the rounding of FP32 distances of the nearest, which
+ * get the smallest such distance. At most
  * CORA_NOALLOC_MAX_CENTROIDS centroids and dimension CORA_NOALLOC_MAX_DIM (else
  * CORA_ERR_INVALID_ARGUMENT). Runs on the null stream and returns when done; calls on one GPU
  * take turns on its scratch array (a per-device lock), so several host threads may call it. */
