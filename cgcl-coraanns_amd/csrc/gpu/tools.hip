@@ -48,11 +48,17 @@ __device__ __forceinline__ float nearest_cut(float best, float xnorm, uint32_t d
     return best + 2.2f * (float)(dim + 34) * 0x1p-24f * r * r;
 }
 
+// Rows of x and cent may be read four values at a time (the callers of cora_tool_assign_noalloc own
+// both arrays, at any alignment).
+__device__ __forceinline__ bool quad_rows(const float *x, const float *cent, uint32_t dim) {
+    return dim % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(cent)) & 15) == 0;
+}
+
 // sum (x - c)^2 in FP64 for N centroids at a time by a group of eight lanes (the same in all of
-// them). Aligned rows of whole quads are read four values at a time.
+// them)
 template <int N>
 __device__ __forceinline__ void group_l2(const float *__restrict__ x, const float *const (&c)[N], uint32_t dim,
-                                         uint32_t gl, double (&s)[N]) {
+                                         bool quads, uint32_t gl, double (&s)[N]) {
 #pragma unroll
     for (int j = 0; j < N; ++j)
         s[j] = 0.0;
@@ -60,7 +66,7 @@ __device__ __forceinline__ void group_l2(const float *__restrict__ x, const floa
         const double d = (double)a - (double)b;
         return fma(d, d, acc);
     };
-    if (dim % 4 == 0) {
+    if (quads) {
         for (uint32_t i = 4 * gl; i < dim; i += 32) {
             const float4 a = *reinterpret_cast<const float4 *>(x + i);
 #pragma unroll
@@ -134,11 +140,12 @@ __global__ __launch_bounds__(64) void row_argmin_kernel(const float *__restrict_
         }
         __syncthreads();
         if (n > 1 && n <= kNearFew) {
+            const bool quads = quad_rows(x, cent, dim);
             double bd = __longlong_as_double(0x7FF0000000000000ll);
             for (uint32_t i = lane / 8; i < n; i += 8) {
                 const float *const c[1] = {cent + (size_t)s_cand[i] * dim};
                 double d[1];
-                group_l2<1>(x + (size_t)blockIdx.x * dim, c, dim, lane & 7, d);
+                group_l2<1>(x + (size_t)blockIdx.x * dim, c, dim, quads, lane & 7, d);
                 if (i < 8 || d[0] < bd || (d[0] == bd && s_cand[i] < bi)) {
                     bd = d[0];
                     bi = s_cand[i];
@@ -232,6 +239,7 @@ __global__ __launch_bounds__(256) void nearest_exact_kernel(const unsigned long 
     __shared__ uint32_t s_item[256], s_whole[256], s_items, s_wholes;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t & 63, group = t / 8, gl = t & 7;
     const uint32_t near = count[0];
+    const bool quads = quad_rows(x, cent, dim);
     const bool crowded = (uint64_t)count[1] * k <= kCrowdedEvals * ((uint64_t)rows + 4096);
     const uint32_t n = near + (crowded ? count[1] : 0u);
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
@@ -275,7 +283,7 @@ __global__ __launch_bounds__(256) void nearest_exact_kernel(const unsigned long 
             for (uint32_t j = group; j < items; j += 32) {
                 const float *const c[1] = {cent + (size_t)s_item[j] * dim};
                 double d[1];
-                group_l2<1>(xr, c, dim, gl, d);
+                group_l2<1>(xr, c, dim, quads, gl, d);
                 take(d[0], s_item[j]);
             }
             for (uint32_t j = 0; j < wholes; ++j) {
@@ -285,7 +293,7 @@ __global__ __launch_bounds__(256) void nearest_exact_kernel(const unsigned long 
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
                     c[u] = cent + (size_t)min(c0 + 32 * u, k - 1) * dim;
-                group_l2<4>(xr, c, dim, gl, d);
+                group_l2<4>(xr, c, dim, quads, gl, d);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
                     if (c0 + 32 * u < k)

@@ -73,6 +73,36 @@ def test_assign_noalloc_matches_assign():
         assert np.array_equal(got, want), (n, dim, k, int((got != want).sum()))
 
 
+def test_assign_noalloc_on_unaligned_arrays():
+    """Rows and centroids that begin one or two floats after an aligned address, with near ties (the
+    FP64 settlement reads the rows again): the FP64 nearest, as on aligned ones."""
+    rt = hip_runtime()
+    assert rt.hipSetDevice(0) == 0
+    gpu = ca._load()[0]
+    rng = np.random.default_rng(8)
+    n, dim, k = 3000, 128, 200
+    c = rng.standard_normal((k, dim)).astype(np.float32)
+    x = (c[rng.integers(0, k, n)] + 0.1 * rng.standard_normal((n, dim))).astype(np.float32)
+    x[:50] = (c[3] + c[90]) / 2
+    c[150] = c[7]
+    x[50:80] = c[7]
+    d = np.stack([((r.astype(np.float64) - c.astype(np.float64)) ** 2).sum(1) for r in x])
+    say("[gpu] assign_noalloc on unaligned arrays")
+    for ox, oc in [(0, 0), (1, 0), (0, 2), (1, 3)]:
+        dx = DeviceArray(rt, np.concatenate([np.zeros(ox, np.float32), x.ravel()]))
+        dc = DeviceArray(rt, np.concatenate([np.zeros(oc, np.float32), c.ravel()]))
+        da = DeviceArray(rt, np.full(n, 0xFFFFFFFF, np.uint32))
+        try:
+            ca._tool_check(gpu.cora_tool_assign_noalloc(C.c_void_p(dx.ptr.value + 4 * ox), n, dim,
+                                                        C.c_void_p(dc.ptr.value + 4 * oc), k, da.ptr, 0))
+            got = da.read().astype(np.int64)
+        finally:
+            for a in (dx, dc, da):
+                a.free()
+        assert np.all(d[np.arange(n), got] <= d.min(1) * (1 + dim * 2.0 ** -50)), (ox, oc)
+        assert not np.any(got == 150)
+
+
 def test_assign_noalloc_rejects_sizes_beyond_its_scratch():
     rt = hip_runtime()
     assert rt.hipSetDevice(0) == 0
