@@ -420,8 +420,10 @@ struct Nearest {
         k = (uint32_t)k_;
         Kp = split_padded(dim_);
         tiles = nearest_tiles(k);
-        // 32-bit element offsets of a chunk's rows, and 1 GiB of tile minima
-        chunk = std::max<size_t>(1, std::min<size_t>({max_rows, ((1ull << 31) - 1) / Kp, (1ull << 30) / (12ull * tiles)}));
+        // 32-bit element offsets of a chunk's rows, 1 GiB of tile minima, and a wave per row within the
+        // 2^32 work-items of a dispatch
+        chunk = std::max<size_t>(1, std::min<size_t>({max_rows, ((1ull << 31) - 1) / Kp, (1ull << 30) / (12ull * tiles),
+                                                      size_t{1} << 25}));
         c.add_to(block, k, Kp);
         block.add(best, chunk * tiles);
         block.add(second, chunk * tiles);
@@ -486,6 +488,12 @@ bool split_or_fp32(DevBlock &split) {
         return true;
     (void)hipGetLastError();
     return false;
+}
+
+// rows whose distances to k centroids the FP32 GEMM forms at a time: 1 GiB of them, and row tiles
+// of 64 within a launch's second dimension
+size_t fp32_chunk_rows(size_t rows, uint64_t k) {
+    return std::max<size_t>(1, std::min<size_t>({rows, (size_t)(1u << 30) / (k * 4), size_t{1} << 21}));
 }
 
 // rows of a chunk that is computed on while the next ones are copied: whole GEMM tiles, 64 MiB
@@ -645,7 +653,7 @@ int cora_tool_kmeans(const float *h_x, uint64_t n, uint64_t dim, uint64_t k, uin
     for (uint64_t i = 0; i < k; ++i)
         memcpy(&init[i * dim], h_x + pick[i] * dim, dim * 4);
     bool split = Nearest::supported(dim, k);
-    const size_t chunk = std::max<size_t>(1, std::min<size_t>(n, (size_t)(1u << 30) / (k * 4)));
+    const size_t chunk = fp32_chunk_rows(n, k);
     DevBlock block, split_block, fp32_block;
     float *x, *c, *sums, *cn, *xn, *dist;
     uint32_t *asg, *cnt;
@@ -718,7 +726,7 @@ int cora_tool_assign(const float *h_x, uint64_t n, uint64_t dim, const float *h_
         return CORA_ERR_INVALID_ARGUMENT;
     TCHK(hipSetDevice(device));
     const size_t rows_dev = std::min<size_t>(n, 1u << 22);
-    const size_t chunk = std::max<size_t>(1, std::min<size_t>(rows_dev, (size_t)(1u << 30) / (k * 4)));
+    const size_t chunk = fp32_chunk_rows(rows_dev, k);
     bool split = Nearest::supported(dim, k);
     DevBlock block, split_block, fp32_block;
     float *x, *c, *cn, *xn, *dist;

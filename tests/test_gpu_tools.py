@@ -194,6 +194,28 @@ def test_topk_l2_beyond_2_32_work_items():
             assert set(want.tolist()) == set(ids[i].tolist())
 
 
+def test_kmeans_beyond_2_32_work_items():
+    """More than 2^32 / 64 rows (67.2M x 8): one 64-lane wave per row in one launch would exceed the
+    dispatch's 32-bit work-item count. Rows of zeros and ones, of 256 kinds, so that the sums are
+    whole numbers below 2^24: after one iteration every centroid is the mean of its rows."""
+    n, dim, k = 67_200_000, 8, 16
+    kinds = ((np.arange(256)[:, None] >> np.arange(8)) & 1).astype(np.float32)
+    kind = np.random.default_rng(67).integers(0, 256, n, dtype=np.uint8)
+    x = kinds[kind]
+    count = np.bincount(kind, minlength=256).astype(np.float64)
+    say(f"[tools] k-means over {n:,} rows")
+    for seed in range(20):
+        c = ca.gpu_kmeans(x, k, 0, seed=seed)
+        a = fp64_scores(c, kinds, 0).argmin(1)  # whole numbers: ties exact, to the lower id
+        rows = np.bincount(a, weights=count, minlength=k)
+        if len(np.unique(c, axis=0)) == k and rows.max() < 2 ** 24:
+            break
+    else:
+        raise AssertionError("no seed with distinct first rows")
+    want = np.stack([np.bincount(a, weights=count * kinds[:, d], minlength=k) for d in range(dim)], 1) / rows[:, None]
+    assert np.abs(ca.gpu_kmeans(x, k, 1, seed=seed) - want).max() < 1e-6
+
+
 @pytest.mark.parametrize("P", [64, 192, 384, 768, 960, 1024])
 @pytest.mark.parametrize("metric", [0, 1])
 def test_quantiser_on_unusual_rows(P, metric):
